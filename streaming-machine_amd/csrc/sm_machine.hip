@@ -13,6 +13,7 @@
 #include "sm_kernels.hip"
 #include "sm_batch.hip"
 #include "sm_attend_split.hip"
+#include "sm_prompt.hip"
 #include "../../include/sm_base2.h"
 
 #include <hip/hip_ext.h>
@@ -352,6 +353,18 @@ static const int NOUT[4] = {2304, 768, 3072, 768};
 static const int TCOLS[4] = {2, 2, 2, 1};      // tile widths: qkv, proj, fc, mproj (one wave per tile)
 static const char* BANK[4] = {"qkv", "proj", "fc", "mproj"};
 
+// The prompt pass in large passes (sm_prompt.hip): its rows' buffers, for cap rows; the streams' own rows (R, QKV,
+// ...) stay the decode steps'.
+#define SM_PROMPT_CAP 4096       // rows a pass at most
+#define SM_PROMPT_CTX 16384      // (k_pattend's int32 sums hold that many positions)
+struct PromptWS {
+    int cap = 0;                                        // 0: no large passes
+    i64 *R = nullptr, *QKV = nullptr, *att = nullptr, *hid = nullptr;      // [cap][768 | 2304 | 768 | 3072]
+    signed char* pl[3] = {};                            // light planes: two of 768-wide rows, one of 3072-wide rows
+    int* ri[3] = {};                                    // their row facts
+    PChunk* ch = nullptr;                               // the attention's chunks [slot][12][chunks]
+};
+
 struct sm_machine {
     sm_config cfg{};
     int B = 1, ctx = 0, vocab = 0, npos = 0, head_grid = 1024;
@@ -436,6 +449,7 @@ struct sm_machine {
     int* pfmap = nullptr;                               // [B][ctx]
     std::vector<int> h_pfmap;
     int h_pfpos = 0;
+    PromptWS pw;
     // host mirror
     int h_plen = 0, h_pos = 0, h_words = 0, h_recpos = -1;
     std::vector<std::vector<int>> prompts;
@@ -543,6 +557,9 @@ static void machine_free(sm_machine* m) {
                   m->top_hi, m->top_lo, m->cand_j, m->cand_h, m->cand_c, m->top_x, m->top_f, m->top_n, m->top_w,
                   m->top_pile, m->top_score, m->asc, m->acm, m->aacc, m->V64, m->VW, m->vbig};
     for (void* p : ps) hfree(p);
+    PromptWS& w = m->pw;
+    void* pp[] = {w.R, w.QKV, w.att, w.hid, w.pl[0], w.pl[1], w.pl[2], w.ri[0], w.ri[1], w.ri[2], w.ch};
+    for (void* p : pp) hfree(p);
     for (int l = 0; l < 12; l++)
         for (int j = 0; j < 2; j++) { hfree(m->ng[l][j]); hfree(m->nb[l][j]); }
     if (m->hpin) (void)hipHostFree(m->hpin);
@@ -1209,6 +1226,89 @@ static int launch_step(sm_machine* m, int parts = STEP_ALL, bool rec = false, bo
     return SM_OK;
 }
 
+// One large pass: positions [pa, pb) of the S streams from s0 (sm_prompt.hip's row order; map: the rows' entries of
+// pfmap).  The last layer only stores its keys and values (the rest feeds the head alone).
+template <int K, int EPI>
+static void pgemm(sm_machine* m, const char* name, const MfmaPlate& P, int set, i64* Y, int rows) {
+    PGemmArgs a{};
+    a.N = P.N; a.rows = rows; a.W = P.W; a.csum = P.csum; a.we = P.e; a.bias = P.b;
+    a.planes = m->pw.pl[set]; a.rowinfo = m->pw.ri[set]; a.Y = Y; a.tb = m->T.tb();
+    a.err = m->kind == 1 ? m->ctl + CTL_ERR : nullptr;
+    const int tiles = (P.N / (16 * PBN)) * ((rows + 16 * PBM - 1) / (16 * PBM));
+    launch(m->cfg.profile, name, k_pgemm<K, EPI>, dim3((tiles + 7) / 8 * 8), dim3(256), 0, m->st, a);
+}
+template <int MODEL>
+static int launch_prompt(sm_machine* m, int s0, int S, int pa, int pb, const int* map) {
+    PromptWS& w = m->pw;
+    const bool timed = m->cfg.profile;
+    const int n = pb - pa, rows = S * n;
+    const Tables tb = m->T.tb();
+    auto light = [&](const i64* X, int set, bool gauged) {
+        LightArgs a{};
+        a.rows = rows; a.X = X; a.Rw = w.R; a.planes = w.pl[set]; a.rowinfo = w.ri[set]; a.tb = tb; a.ls_row = gauged;
+        a.wte = m->wte; a.wpe = m->wpe; a.seq = m->seq; a.seq_stride = m->ctx + 1; a.rowmap = map;
+        return a;
+    };
+    auto to16 = [&](const char* name, const i64* X, int set) {
+        if (set == 2) launch(timed, name, k_light<3072, PRO_TO16, 768, 1>, dim3(rows), dim3(768), 0, m->st, light(X, set, false));
+        else launch(timed, name, k_light<768, PRO_TO16, 192, 1>, dim3(rows), dim3(192), 0, m->st, light(X, set, false));
+    };
+    // the stream rows' gauges for layer l (l < 0: the words enter first)
+    auto gauge = [&](int l) {
+        if constexpr (MODEL == 1) {
+            PyRowArgs a{};
+            const int g = l < 0 ? 0 : l;
+            a.err = m->ctl + CTL_ERR; a.rows = rows; a.R = w.R; a.ew = m->ew; a.ee = m->ee; a.seq = m->seq;
+            a.seq_stride = m->ctx + 1; a.tb = tb; a.rowmap = map;
+            a.ng1 = m->ng[g][0]; a.nb1 = m->nb[g][0]; a.nge1 = m->nge[g][0]; a.planes1 = w.pl[0]; a.rowinfo1 = w.ri[0];
+            a.ng2 = m->ng[g][1]; a.nb2 = m->nb[g][1]; a.nge2 = m->nge[g][1]; a.planes2 = w.pl[1]; a.rowinfo2 = w.ri[1];
+            if (l < 0) launch(timed, "prompt.embed", k_py_rows<PY_EMBED>, dim3(rows), dim3(192), 0, m->st, a);
+            else launch(timed, "prompt.gauge", k_py_rows<PY_GAUGE>, dim3(rows), dim3(192), 0, m->st, a);
+        } else if (l < 0) {
+            launch(timed, "prompt.embed", k_light<768, PRO_EMBED, 192, 1>, dim3(rows), dim3(192), 0, m->st, light(nullptr, 0, true));
+        } else {
+            launch(timed, "prompt.gauge", k_light<768, PRO_GAUGE, 192, 1>, dim3(rows), dim3(192), 0, m->st, light(w.R, 0, true));
+        }
+    };
+    gauge(-1);
+    for (int l = 0; l < 12; l++) {
+        const MfmaPlate* P = m->mbank[l];
+        pgemm<768, MODEL == 1 ? EPI_PLAIN : EPI_GAUGED>(m, "prompt.qkv", P[0], 0, w.QKV, rows);
+        PAttArgs g{};
+        AttArgs& a = g.a;
+        const size_t per = (size_t)m->B * m->ctx;
+        a.QKV = w.QKV; a.K16 = m->K16 + l * per * 768; a.KM = m->KM + l * per * 12; a.EK = m->EK + l * per * 12;
+        a.V = m->V + l * per * 768; a.V64 = m->V64 ? m->V64 + l * per * 768 : nullptr;
+        a.VW = m->VW ? m->VW + l * per * 12 : nullptr; a.vbig = m->vbig ? m->vbig + (size_t)l * m->B * 12 : nullptr;
+        a.out = w.att; a.ctx = m->ctx; a.tb = tb; a.err = m->ctl + CTL_ERR; a.rowmap = map;
+        a.cosT = m->cosT; a.sinT = m->sinT; a.rot = m->rot; a.half = m->half; a.ehalf = m->ehalf;
+        if (l == 11) {
+            launch(timed, "prompt.kv", k_kv_rows<MODEL>, dim3(12, rows), dim3(128), 0, m->st, a);
+            break;
+        }
+        if constexpr (MODEL == 1) {                    // the other half of the parallel residual, to its light
+            pgemm<768, EPI_PLAIN_EDGE>(m, "prompt.fc", P[2], 1, w.hid, rows);
+            to16("prompt.light.hid", w.hid, 2);
+        }
+        g.ch = w.ch; g.n = n; g.pa = pa; g.pb = pb; g.s0 = s0; g.nch = (pb + PCH - 1) / PCH;
+        launch(timed, "prompt.chunks", k_kv_chunk<MODEL>, dim3(g.nch, 12, S), dim3(256), 0, m->st, g);
+        const dim3 qt((n + 15) / 16, 12, S);
+        if (g.nch > 1) launch(timed, "prompt.attend", k_pattend<MODEL, 4>, qt, dim3(256), 0, m->st, g);
+        else launch(timed, "prompt.attend", k_pattend<MODEL, 1>, qt, dim3(64), 0, m->st, g);
+        to16("prompt.light.att", w.att, 0);
+        pgemm<768, EPI_PLAIN_ADD>(m, "prompt.proj", P[1], 0, w.R, rows);
+        if constexpr (MODEL == 0) {
+            gauge(l);                                  // (GPT-2's two norms are folded into their plates)
+            pgemm<768, EPI_GAUGED_EDGE>(m, "prompt.fc", P[2], 0, w.hid, rows);
+            to16("prompt.light.hid", w.hid, 2);
+        }
+        pgemm<3072, EPI_PLAIN_ADD>(m, "prompt.mproj", P[3], 2, w.R, rows);
+        gauge(l + 1);
+    }
+    HIP_TRY(hipGetLastError());
+    return SM_OK;
+}
+
 // positions [0, npos) of every stream as passes of up to prefill_rows prompt rows, stream by stream (rows of one
 // stream in position order, so a pass's keys and values at earlier positions are cached before it runs); then the
 // device position moves to npos.  Nothing is recorded: the caller stops short of a recorded position.
@@ -1218,7 +1318,19 @@ static int run_prefill(sm_machine* m, int npos) {
     for (int s = 0; s < m->B; s++)
         for (int q = 0; q < npos; q++) m->h_pfmap[(size_t)s * npos + q] = s << 16 | q;
     HIP_TRY(hipMemcpyAsync(m->pfmap, m->h_pfmap.data(), (size_t)total * 4, hipMemcpyHostToDevice, m->st));
-    for (int r0 = 0; r0 < total; r0 += chunk) {
+    const bool large = m->pw.cap > 0 && total > chunk;
+    if (large) {
+        // whole prompts of as many streams as fit, or a prompt longer than the buffers in parts
+        const int per = std::min(m->B, std::max(1, m->pw.cap / npos)), step = std::min(npos, m->pw.cap);
+        for (int s = 0; s < m->B; s += per)
+            for (int q = 0; q < npos; q += step) {
+                const int S = std::min(per, m->B - s), e = std::min(npos, q + step);
+                const int* map = m->pfmap + (size_t)s * npos + q;
+                const int rc = m->kind == 1 ? launch_prompt<1>(m, s, S, q, e, map) : launch_prompt<0>(m, s, S, q, e, map);
+                if (rc) return rc;
+            }
+    }
+    for (int r0 = 0; r0 < total && !large; r0 += chunk) {
         const int n = std::min(chunk, total - r0), RT = (n + 15) / 16;
         const int* map = m->pfmap + r0;
         int rc;
@@ -1477,6 +1589,19 @@ extern "C" int sm_create(const char* layout_dir, const sm_config* cfg, sm_machin
         (rc = dalloc(&m->r_logits, (size_t)m->vocab)) || (rc = dalloc(&m->r_gauge, (size_t)12 * 2 * 768)) ||
         (rc = dalloc(&m->r_fcpre, (size_t)12 * 3072)) || (rc = dalloc(&m->r_hgauge, (size_t)768)))
         return bail(rc);
+    // the large prompt passes' buffers (prefill_rows 64, where a prompt can hold more rows than one small pass)
+    if (mfma && c.prefill_rows == 64 && B * (ctx - 1) > 64 && ctx <= SM_PROMPT_CTX) {
+        PromptWS& w = m->pw;
+        const size_t cap = std::min<size_t>(SM_PROMPT_CAP, (B * (ctx - 1) + 127) / 128 * 128);
+        const size_t nch = std::max((cap + 63 * B) / PCH + 1, (ctx + PCH - 1) / PCH);
+        if ((rc = dalloc(&w.R, cap * 768)) || (rc = dalloc(&w.QKV, cap * 2304)) || (rc = dalloc(&w.att, cap * 768)) ||
+            (rc = dalloc(&w.hid, cap * 3072)) || (rc = dalloc(&w.pl[0], cap * 768 * 3)) ||
+            (py && (rc = dalloc(&w.pl[1], cap * 768 * 3))) || (rc = dalloc(&w.pl[2], cap * 3072 * 3)) ||
+            (rc = dalloc(&w.ri[0], cap * 8)) || (rc = dalloc(&w.ri[1], cap * 8)) || (rc = dalloc(&w.ri[2], cap * 8)) ||
+            (rc = dalloc(&w.ch, nch * 12)))
+            return bail(rc);
+        w.cap = (int)cap;
+    }
     // rows with a value past 32 bits whole beside their low 32 bits (the float arrival keeps the int32 cache and its
     // error)
     if (!m->farr && ((rc = dalloc(&m->V64, 12 * B * ctx * 768)) || (rc = dalloc(&m->VW, 12 * B * ctx * 12)) ||

@@ -110,7 +110,8 @@ class Machine:
     Machine(layout_dir, max_ctx=1024, max_streams=1, use_graph=True, prefill_rows=64, gauge="int", edge="int",
             arrival="int")
       prefill_rows: every prompt position but the last goes through the int8 MFMA banks that many rows a pass
-      (base2_stream.swift:274: the prompt through each layer at once); 0 runs it position by position.
+      (base2_stream.swift:274: the prompt through each layer at once; at 64, the default, longer prompts take passes
+      of up to 4096 rows); 0 runs it position by position.
       inv: the complement machine (base2_stream.swift:26 `inv`): stream, plates and lights held bit-complemented on
       the device; the same words (GPT-2, one stream, prefill_rows=0).
       top: "fr" (base2_stream_fr.swift's collapsing top read: the high bytes of every word, then the low bytes of
