@@ -1,0 +1,51 @@
+"""sm_stage_race over many blocks (more than 16,384 values): the largest value, ties to the lowest index
+(base2.py:34-40), at the sizes where the block count and width change, on values that tie across blocks, that are all
+the type's lowest, and with the index written over the values."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def race(sm, v, out=None, stream=0):
+    d = torch.from_numpy(v).cuda()
+    o = torch.full((1,), 77, dtype=torch.int64, device="cuda")
+    ptr = o.data_ptr() if out is None else d.data_ptr() + 8 * out
+    sm.stages.race(d.data_ptr(), len(v), ptr, stream=stream)
+    torch.cuda.synchronize()
+    return int(o[0]) if out is None else int(d[out])
+
+
+@pytest.mark.parametrize("n", [16384, 16385, 18431, 18433, 131072, 131073, 1048577, 2100001])
+def test_many_blocks(sm, n):
+    rng = np.random.default_rng(n)
+    v = rng.integers(-2 ** 62, 2 ** 62, n)
+    assert race(sm, v) == int(v.argmax())
+    v[[n - 1, n // 2, n // 3, 5000]] = 2 ** 62 + 1             # the same best in several blocks
+    assert race(sm, v) == 5000
+    v[0] = v[n - 1] = np.iinfo(np.int64).max
+    assert race(sm, v) == 0
+    assert race(sm, np.full(n, np.iinfo(np.int64).min)) == 0
+    low = np.full(n, np.iinfo(np.int64).min)
+    low[n - 1] += 1
+    assert race(sm, low) == n - 1
+    assert race(sm, v, out=n // 2) == 0                        # the index over a value: written after it is read
+
+
+def test_two_streams(sm):
+    """races on two streams at once, each with its own winner"""
+    rng = np.random.default_rng(5)
+    vs = [rng.integers(-2 ** 40, 2 ** 40, 50257) for _ in range(2)]
+    ds = [torch.from_numpy(v).cuda() for v in vs]
+    outs = torch.zeros(2, 50, dtype=torch.int64, device="cuda")
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    torch.cuda.synchronize()
+    for i in range(50):
+        for k, s in enumerate(streams):
+            sm.stages.race(ds[k].data_ptr(), 50257, outs[k, i:].data_ptr(), stream=s.cuda_stream)
+    torch.cuda.synchronize()
+    for k in range(2):
+        assert (outs[k] == int(vs[k].argmax())).all()
