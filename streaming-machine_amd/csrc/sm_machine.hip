@@ -280,12 +280,15 @@ struct sm_tables {
     int alen = 0;
     i64 log768 = 0, eps40 = 0;
     int verified = 0;         // every entry equals its defining formula (checked on the device at create)
-    int* scratch = nullptr;   // [0] pos for sm_stage_attend, [1] error bits, [4..7] mismatch counts
+    int* scratch = nullptr;   // [1] error bits, [4..7] mismatch counts
+    int* posn = nullptr;      // [SM_STAGE_ATT_CTX] the numbers 0, 1, ..: the attention entry points' positions
+    int* herr = nullptr;      // pinned host memory: their error bits
     // sm_stage_attend_split's score row, chunk maxima and accumulators (made at its first call, for ctx <= 8192)
     i64 *asc = nullptr, *acm = nullptr, *aacc = nullptr;
     Tables tb() const { return Tables{LOG2, EXP2, PHI, ARR, alen, log768, eps40, GPOW, HPOW, PGPOW}; }
 };
 
+#define SM_STAGE_ATT_CTX 8192      // positions of the attention entry points
 static int upload_table(int** dst, const i64* src, size_t n, i64 lo, i64 hi, const char* name) {
     std::vector<int> v(n);
     for (size_t i = 0; i < n; i++) {
@@ -322,6 +325,16 @@ static int tables_init(sm_tables& T, const i64* phi, const i64* arr, int alen, c
     }
     if ((rc = dalloc(&T.scratch, 16))) return rc;
     HIP_TRY(hipMemset(T.scratch, 0, 64));
+    {
+        std::vector<int> n(SM_STAGE_ATT_CTX);
+        for (int i = 0; i < SM_STAGE_ATT_CTX; i++) n[i] = i;
+        if ((rc = dalloc(&T.posn, n.size()))) return rc;
+        HIP_TRY(hipMemcpy(T.posn, n.data(), n.size() * 4, hipMemcpyHostToDevice));
+        if (hipHostMalloc(&T.herr, 64, hipHostMallocDefault) != hipSuccess) {
+            T.herr = nullptr;
+            return fail(SM_E_OOM, "hipHostMalloc: the error word");
+        }
+    }
     T.alen = alen; T.log768 = log768; T.eps40 = eps40;
     // every entry against its formula (table_mode 1 refuses tables that are not the reference's)
     const int n = alen + 1 > 65536 ? alen + 1 : 65536;
@@ -335,7 +348,8 @@ static int tables_init(sm_tables& T, const i64* phi, const i64* arr, int alen, c
 
 static void tables_free(sm_tables& T) {
     hfree(T.LOG2); hfree(T.EXP2); hfree(T.PHI); hfree(T.ARR); hfree(T.GPOW); hfree(T.HPOW); hfree(T.PGPOW); hfree(T.scratch);
-    hfree(T.asc); hfree(T.acm); hfree(T.aacc);
+    hfree(T.asc); hfree(T.acm); hfree(T.aacc); hfree(T.posn);
+    if (T.herr) (void)hipHostFree(T.herr);
     T = sm_tables();
 }
 
@@ -2037,31 +2051,34 @@ extern "C" int sm_stage_race(const int64_t* v, int64_t n, int64_t* out_index, vo
     HIP_TRY(hipGetLastError());
     return SM_OK;
 }
+// The attention entry points' end: the launched kernels done, and the error they report.  A call is its launches, one
+// copy of the error word into pinned memory and one wait: the position is an entry of a device array of numbers (a
+// copy and a wait of its own before the launch, and the error word into pageable memory, made a call of 9 us of
+// kernels take 47 us).
+static int stage_attend_end(const sm_tables* t, hipStream_t s, const char* what) {
+    HIP_TRY(hipMemcpyAsync(t->herr, t->scratch + 1, 4, hipMemcpyDeviceToHost, s));
+    HIP_TRY(hipStreamSynchronize(s));
+    if (*static_cast<volatile int*>(t->herr) & SM_ERR_V32) {
+        HIP_TRY(hipMemset(t->scratch + 1, 0, 4));
+        return fail(SM_E_OVERFLOW, what);
+    }
+    return SM_OK;
+}
 extern "C" int sm_stage_attend(const sm_tables* t, const int64_t* qkv, int16_t* k16, int64_t* km, int32_t* ek, int32_t* v,
                                int32_t pos, int32_t ctx, int64_t* out, void* stream) {
     if (!t || !qkv || !k16 || !km || !ek || !v || !out || ctx <= 0 || pos < 0 || pos >= ctx || ctx > 8192)
         return fail(SM_E_ARG, "sm_stage_attend: arguments");
     hipStream_t s = (hipStream_t)stream;
-    HIP_TRY(hipMemcpyAsync(t->scratch, &pos, 4, hipMemcpyHostToDevice, s));
-    HIP_TRY(hipStreamSynchronize(s));
     AttArgs a{};
-    a.QKV = (const i64*)qkv; a.K16 = k16; a.KM = (i64*)km; a.EK = ek; a.V = v; a.out = (i64*)out; a.pos = t->scratch; a.ctx = ctx;
+    a.QKV = (const i64*)qkv; a.K16 = k16; a.KM = (i64*)km; a.EK = ek; a.V = v; a.out = (i64*)out; a.pos = t->posn + pos; a.ctx = ctx;
     a.tb = t->tb(); a.err = t->scratch + 1;
     launch(g_kt.stages, "stage.attend", k_attend<0, 1, 0>, dim3(12, 1), dim3(NTHR), (size_t)ctx * 12, s, a);
     HIP_TRY(hipGetLastError());
-    int err = 0;
-    HIP_TRY(hipMemcpyAsync(&err, t->scratch + 1, 4, hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
-    if (err & SM_ERR_V32) {
-        HIP_TRY(hipMemset(t->scratch + 1, 0, 4));
-        return fail(SM_E_OVERFLOW, "sm_stage_attend: a value left 32 bits");
-    }
-    return SM_OK;
+    return stage_attend_end(t, s, "sm_stage_attend: a value left 32 bits");
 }
 
 // the same attention spread over chunks of 64 positions, the batch-1 machine's kernels for positions from its split
 // position on (sm_attend_split.hip)
-#define SM_STAGE_ATT_CTX 8192
 extern "C" int sm_stage_attend_split(const sm_tables* t, const int64_t* qkv, int16_t* k16, int64_t* km, int32_t* ek,
                                      int32_t* v, int32_t pos, int32_t ctx, int64_t* out, void* stream) {
     if (!t || !qkv || !k16 || !km || !ek || !v || !out || ctx <= 0 || pos < 0 || pos >= ctx || ctx > SM_STAGE_ATT_CTX)
@@ -2078,10 +2095,8 @@ extern "C" int sm_stage_attend_split(const sm_tables* t, const int64_t* qkv, int
         }
     }
     hipStream_t s = (hipStream_t)stream;
-    HIP_TRY(hipMemcpyAsync(t->scratch, &pos, 4, hipMemcpyHostToDevice, s));
-    HIP_TRY(hipStreamSynchronize(s));
     AttArgs a{};
-    a.QKV = (const i64*)qkv; a.K16 = k16; a.KM = (i64*)km; a.EK = ek; a.V = v; a.out = (i64*)out; a.pos = t->scratch; a.ctx = ctx;
+    a.QKV = (const i64*)qkv; a.K16 = k16; a.KM = (i64*)km; a.EK = ek; a.V = v; a.out = (i64*)out; a.pos = t->posn + pos; a.ctx = ctx;
     a.tb = t->tb(); a.err = t->scratch + 1;
     a.asc = tt->asc; a.acm = tt->acm; a.aacc = tt->aacc; a.ncm = ncm;
     const dim3 grid(12, (ctx + ACH_SPLIT - 1) / ACH_SPLIT);
@@ -2090,14 +2105,7 @@ extern "C" int sm_stage_attend_split(const sm_tables* t, const int64_t* qkv, int
     launch(timed, "stage.attend.mix", k_att_mix<0, 0>, grid, dim3(256), 0, s, a);
     launch(timed, "stage.attend.finish", k_att_finish<0, 0>, dim3(12), dim3(64), 0, s, a);
     HIP_TRY(hipGetLastError());
-    int err = 0;
-    HIP_TRY(hipMemcpyAsync(&err, t->scratch + 1, 4, hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
-    if (err & SM_ERR_V32) {
-        HIP_TRY(hipMemset(t->scratch + 1, 0, 4));
-        return fail(SM_E_OVERFLOW, "sm_stage_attend_split: a value left 32 bits");
-    }
-    return SM_OK;
+    return stage_attend_end(t, s, "sm_stage_attend_split: a value left 32 bits");
 }
 
 extern "C" int sm_stage_attend_rows(const sm_tables* t, const int64_t* qkv, int32_t rows, int16_t* k16, int64_t* km,
@@ -2106,21 +2114,12 @@ extern "C" int sm_stage_attend_rows(const sm_tables* t, const int64_t* qkv, int3
         ctx > 8192)
         return fail(SM_E_ARG, "sm_stage_attend_rows: arguments");
     hipStream_t s = (hipStream_t)stream;
-    HIP_TRY(hipMemcpyAsync(t->scratch, &pos, 4, hipMemcpyHostToDevice, s));
-    HIP_TRY(hipStreamSynchronize(s));
     AttArgs a{};
-    a.QKV = (const i64*)qkv; a.K16 = k16; a.KM = (i64*)km; a.EK = ek; a.V = v; a.out = (i64*)out; a.pos = t->scratch; a.ctx = ctx;
+    a.QKV = (const i64*)qkv; a.K16 = k16; a.KM = (i64*)km; a.EK = ek; a.V = v; a.out = (i64*)out; a.pos = t->posn + pos; a.ctx = ctx;
     a.tb = t->tb(); a.err = t->scratch + 1;
     launch(g_kt.stages, "stage.attend_rows", k_attend<0, 0, 1>, dim3(12, rows), dim3(NTHR), (size_t)ctx * 12, s, a);      // the batched machine's kernel
     HIP_TRY(hipGetLastError());
-    int err = 0;
-    HIP_TRY(hipMemcpyAsync(&err, t->scratch + 1, 4, hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
-    if (err & SM_ERR_V32) {
-        HIP_TRY(hipMemset(t->scratch + 1, 0, 4));
-        return fail(SM_E_OVERFLOW, "sm_stage_attend_rows: a value left 32 bits");
-    }
-    return SM_OK;
+    return stage_attend_end(t, s, "sm_stage_attend_rows: a value left 32 bits");
 }
 
 // tile_cols > 0: a GEMV plate (one light row per product); tile_cols == 0: an MFMA plate (rows of lights) with
