@@ -1288,8 +1288,6 @@ __global__ __launch_bounds__(256) void k_part_piles(GemmArgs a) {
 BINST_L(768, PRO_EMBED, 1)
 BINST_L(768, PRO_RACE_EMBED, 1)
 BINST_L(768, PRO_GAUGE, 1)
-BINST_L(768, PRO_TO16, 1)
-BINST_L(3072, PRO_TO16, 1)
 BINST_L(768, PRO_X16, 1)
 BINST_L(3072, PRO_X16, 1)
 BINST_L(768, PRO_ADD_GAUGE, 4)

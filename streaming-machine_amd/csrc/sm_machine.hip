@@ -373,7 +373,8 @@ static const char* BANK[4] = {"qkv", "proj", "fc", "mproj"};
 #define SM_PROMPT_CTX 16384      // (k_pattend's int32 sums hold that many positions)
 struct PromptWS {
     int cap = 0;                                        // 0: no large passes
-    i64 *R = nullptr, *QKV = nullptr, *att = nullptr, *hid = nullptr;      // [cap][768 | 2304 | 768 | 3072]
+    i64* R = nullptr;                                   // [cap][768] the stream rows
+    PRow qkv{}, att{}, hid{};                           // [cap][2304 | 768 | 3072]
     signed char* pl[3] = {};                            // light planes: two of 768-wide rows, one of 3072-wide rows
     int* ri[3] = {};                                    // their row facts
     PChunk* ch = nullptr;                               // the attention's chunks [slot][12][chunks]
@@ -572,7 +573,7 @@ static void machine_free(sm_machine* m) {
                   m->top_pile, m->top_score, m->asc, m->acm, m->aacc, m->V64, m->VW, m->vbig};
     for (void* p : ps) hfree(p);
     PromptWS& w = m->pw;
-    void* pp[] = {w.R, w.QKV, w.att, w.hid, w.pl[0], w.pl[1], w.pl[2], w.ri[0], w.ri[1], w.ri[2], w.ch};
+    void* pp[] = {w.R, w.qkv.x32, w.qkv.x64, w.qkv.orw, w.att.x32, w.att.x64, w.att.orw, w.hid.x32, w.hid.x64, w.hid.orw, w.pl[0], w.pl[1], w.pl[2], w.ri[0], w.ri[1], w.ri[2], w.ch};
     for (void* p : pp) hfree(p);
     for (int l = 0; l < 12; l++)
         for (int j = 0; j < 2; j++) { hfree(m->ng[l][j]); hfree(m->nb[l][j]); }
@@ -1243,13 +1244,13 @@ static int launch_step(sm_machine* m, int parts = STEP_ALL, bool rec = false, bo
 // One large pass: positions [pa, pb) of the S streams from s0 (sm_prompt.hip's row order; map: the rows' entries of
 // pfmap).  The last layer only stores its keys and values (the rest feeds the head alone).
 template <int K, int EPI>
-static void pgemm(sm_machine* m, const char* name, const MfmaPlate& P, int set, i64* Y, int rows) {
+static void pgemm(sm_machine* m, const char* name, const MfmaPlate& P, int set, i64* Y, const PRow& y, int rows) {
     PGemmArgs a{};
     a.N = P.N; a.rows = rows; a.W = P.W; a.csum = P.csum; a.we = P.e; a.bias = P.b;
-    a.planes = m->pw.pl[set]; a.rowinfo = m->pw.ri[set]; a.Y = Y; a.tb = m->T.tb();
+    a.planes = m->pw.pl[set]; a.rowinfo = m->pw.ri[set]; a.Y = Y; a.y = y; a.tb = m->T.tb();
     a.err = m->kind == 1 ? m->ctl + CTL_ERR : nullptr;
-    const int tiles = (P.N / (16 * PBN)) * ((rows + 16 * PBM - 1) / (16 * PBM));
-    launch(m->cfg.profile, name, k_pgemm<K, EPI>, dim3((tiles + 7) / 8 * 8), dim3(256), 0, m->st, a);
+    const int grid = ((P.ntiles + 3) / 4) * ((rows + 63) / 64);
+    launch(m->cfg.profile, name, k_pgemm<K, EPI, 4, 4, 2, 2, 2>, dim3((grid + 7) / 8 * 8), dim3(256), 0, m->st, a);
 }
 template <int MODEL>
 static int launch_prompt(sm_machine* m, int s0, int S, int pa, int pb, const int* map) {
@@ -1257,15 +1258,12 @@ static int launch_prompt(sm_machine* m, int s0, int S, int pa, int pb, const int
     const bool timed = m->cfg.profile;
     const int n = pb - pa, rows = S * n;
     const Tables tb = m->T.tb();
-    auto light = [&](const i64* X, int set, bool gauged) {
-        LightArgs a{};
-        a.rows = rows; a.X = X; a.Rw = w.R; a.planes = w.pl[set]; a.rowinfo = w.ri[set]; a.tb = tb; a.ls_row = gauged;
+    const dim3 lgrid((rows + 7) / 8);
+    auto light = [&](const i64* X, const PRow& x, int set) {
+        PLightArgs a{};
+        a.rows = rows; a.X = X; a.x = x; a.Rw = w.R; a.planes = w.pl[set]; a.rowinfo = w.ri[set]; a.tb = tb;
         a.wte = m->wte; a.wpe = m->wpe; a.seq = m->seq; a.seq_stride = m->ctx + 1; a.rowmap = map;
         return a;
-    };
-    auto to16 = [&](const char* name, const i64* X, int set) {
-        if (set == 2) launch(timed, name, k_light<3072, PRO_TO16, 768, 1>, dim3(rows), dim3(768), 0, m->st, light(X, set, false));
-        else launch(timed, name, k_light<768, PRO_TO16, 192, 1>, dim3(rows), dim3(192), 0, m->st, light(X, set, false));
     };
     // the stream rows' gauges for layer l (l < 0: the words enter first)
     auto gauge = [&](int l) {
@@ -1279,44 +1277,45 @@ static int launch_prompt(sm_machine* m, int s0, int S, int pa, int pb, const int
             if (l < 0) launch(timed, "prompt.embed", k_py_rows<PY_EMBED>, dim3(rows), dim3(192), 0, m->st, a);
             else launch(timed, "prompt.gauge", k_py_rows<PY_GAUGE>, dim3(rows), dim3(192), 0, m->st, a);
         } else if (l < 0) {
-            launch(timed, "prompt.embed", k_light<768, PRO_EMBED, 192, 1>, dim3(rows), dim3(192), 0, m->st, light(nullptr, 0, true));
+            launch(timed, "prompt.embed", k_plight<768, PRO_EMBED, 64>, lgrid, dim3(512), 0, m->st, light(nullptr, PRow{}, 0));
         } else {
-            launch(timed, "prompt.gauge", k_light<768, PRO_GAUGE, 192, 1>, dim3(rows), dim3(192), 0, m->st, light(w.R, 0, true));
+            launch(timed, "prompt.gauge", k_plight<768, PRO_GAUGE, 64>, lgrid, dim3(512), 0, m->st, light(w.R, PRow{}, 0));
         }
     };
     gauge(-1);
     for (int l = 0; l < 12; l++) {
         const MfmaPlate* P = m->mbank[l];
-        pgemm<768, MODEL == 1 ? EPI_PLAIN : EPI_GAUGED>(m, "prompt.qkv", P[0], 0, w.QKV, rows);
+        pgemm<768, MODEL == 1 ? EPI_PLAIN : EPI_GAUGED>(m, "prompt.qkv", P[0], 0, nullptr, w.qkv, rows);
         PAttArgs g{};
         AttArgs& a = g.a;
         const size_t per = (size_t)m->B * m->ctx;
-        a.QKV = w.QKV; a.K16 = m->K16 + l * per * 768; a.KM = m->KM + l * per * 12; a.EK = m->EK + l * per * 12;
+        a.K16 = m->K16 + l * per * 768; a.KM = m->KM + l * per * 12; a.EK = m->EK + l * per * 12;
         a.V = m->V + l * per * 768; a.V64 = m->V64 ? m->V64 + l * per * 768 : nullptr;
         a.VW = m->VW ? m->VW + l * per * 12 : nullptr; a.vbig = m->vbig ? m->vbig + (size_t)l * m->B * 12 : nullptr;
-        a.out = w.att; a.ctx = m->ctx; a.tb = tb; a.err = m->ctl + CTL_ERR; a.rowmap = map;
+        a.ctx = m->ctx; a.tb = tb; a.err = m->ctl + CTL_ERR;
         a.cosT = m->cosT; a.sinT = m->sinT; a.rot = m->rot; a.half = m->half; a.ehalf = m->ehalf;
-        if (l == 11) {
-            launch(timed, "prompt.kv", k_kv_rows<MODEL>, dim3(12, rows), dim3(128), 0, m->st, a);
+        g.x = w.qkv; g.out = w.att; g.ch = l < 11 ? w.ch : nullptr;
+        g.n = n; g.pa = pa; g.pb = pb; g.s0 = s0; g.nch = (pb + PCH - 1) / PCH;
+        if (l == 11) {                                 // (the pass's own chunks)
+            launch(timed, "prompt.kv", k_kv_chunk<MODEL>, dim3(g.nch, 12, S), dim3(1024), 0, m->st, g);
             break;
         }
         if constexpr (MODEL == 1) {                    // the other half of the parallel residual, to its light
-            pgemm<768, EPI_PLAIN_EDGE>(m, "prompt.fc", P[2], 1, w.hid, rows);
-            to16("prompt.light.hid", w.hid, 2);
+            pgemm<768, EPI_PLAIN_EDGE>(m, "prompt.fc", P[2], 1, nullptr, w.hid, rows);
+            launch(timed, "prompt.light.hid", k_plight<3072, PRO_TO16, PSW>, lgrid, dim3(512), 0, m->st, light(nullptr, w.hid, 2));
         }
-        g.ch = w.ch; g.n = n; g.pa = pa; g.pb = pb; g.s0 = s0; g.nch = (pb + PCH - 1) / PCH;
-        launch(timed, "prompt.chunks", k_kv_chunk<MODEL>, dim3(g.nch, 12, S), dim3(256), 0, m->st, g);
+        launch(timed, "prompt.chunks", k_kv_chunk<MODEL>, dim3(g.nch, 12, S), dim3(1024), 0, m->st, g);
         const dim3 qt((n + 15) / 16, 12, S);
         if (g.nch > 1) launch(timed, "prompt.attend", k_pattend<MODEL, 4>, qt, dim3(256), 0, m->st, g);
         else launch(timed, "prompt.attend", k_pattend<MODEL, 1>, qt, dim3(64), 0, m->st, g);
-        to16("prompt.light.att", w.att, 0);
-        pgemm<768, EPI_PLAIN_ADD>(m, "prompt.proj", P[1], 0, w.R, rows);
+        launch(timed, "prompt.light.att", k_plight<768, PRO_TO16, 64>, lgrid, dim3(512), 0, m->st, light(nullptr, w.att, 0));
+        pgemm<768, EPI_PLAIN_ADD>(m, "prompt.proj", P[1], 0, w.R, PRow{}, rows);
         if constexpr (MODEL == 0) {
             gauge(l);                                  // (GPT-2's two norms are folded into their plates)
-            pgemm<768, EPI_GAUGED_EDGE>(m, "prompt.fc", P[2], 0, w.hid, rows);
-            to16("prompt.light.hid", w.hid, 2);
+            pgemm<768, EPI_GAUGED_EDGE>(m, "prompt.fc", P[2], 0, nullptr, w.hid, rows);
+            launch(timed, "prompt.light.hid", k_plight<3072, PRO_TO16, PSW>, lgrid, dim3(512), 0, m->st, light(nullptr, w.hid, 2));
         }
-        pgemm<3072, EPI_PLAIN_ADD>(m, "prompt.mproj", P[3], 2, w.R, rows);
+        pgemm<3072, EPI_PLAIN_ADD>(m, "prompt.mproj", P[3], 2, w.R, PRow{}, rows);
         gauge(l + 1);
     }
     HIP_TRY(hipGetLastError());
@@ -1608,8 +1607,13 @@ extern "C" int sm_create(const char* layout_dir, const sm_config* cfg, sm_machin
         PromptWS& w = m->pw;
         const size_t cap = std::min<size_t>(SM_PROMPT_CAP, (B * (ctx - 1) + 127) / 128 * 128);
         const size_t nch = std::max((cap + 63 * B) / PCH + 1, (ctx + PCH - 1) / PCH);
-        if ((rc = dalloc(&w.R, cap * 768)) || (rc = dalloc(&w.QKV, cap * 2304)) || (rc = dalloc(&w.att, cap * 768)) ||
-            (rc = dalloc(&w.hid, cap * 3072)) || (rc = dalloc(&w.pl[0], cap * 768 * 3)) ||
+        auto prow = [&](PRow& r, size_t n, size_t sw) -> int {
+            int e;
+            if ((e = dalloc(&r.x32, cap * n)) || (e = dalloc(&r.x64, cap * n)) || (e = dalloc(&r.orw, cap * n / sw))) return e;
+            return SM_OK;
+        };
+        if ((rc = dalloc(&w.R, cap * 768)) || (rc = prow(w.qkv, 2304, PSW)) || (rc = prow(w.att, 768, 64)) ||
+            (rc = prow(w.hid, 3072, PSW)) || (rc = dalloc(&w.pl[0], cap * 768 * 3)) ||
             (py && (rc = dalloc(&w.pl[1], cap * 768 * 3))) || (rc = dalloc(&w.pl[2], cap * 3072 * 3)) ||
             (rc = dalloc(&w.ri[0], cap * 8)) || (rc = dalloc(&w.ri[1], cap * 8)) || (rc = dalloc(&w.ri[2], cap * 8)) ||
             (rc = dalloc(&w.ch, nch * 12)))
