@@ -2200,9 +2200,19 @@ static void rows_product(const sm_plate* p, const int64_t* x16, int32_t rows, in
     ga.planes = planes; ga.rowinfo = rowinfo; ga.Y = (i64*)pile; ga.ystride = P.N;
     if (P.K == 768) {
         launch(timed, "plate.light", k_light<768, PRO_X16, 192, 1>, dim3(rows), dim3(192), 0, s, la);
-        if (P.N > 3072)       // head-shaped plates: the head's kernel (light planes in LDS)
+        // head-shaped plates.  From 16,000 columns (32 rows at most; 36,000 for more) the prompt passes' bank, a block 64
+        // columns of every row; below, where that leaves CUs idle, the head's kernel.  Back to back, this bank / that
+        // kernel: 16 rows 11.1 / 12.6 us at 16,000 columns, 25.6 / 27.5 at 50,257; 32 rows 13.2 / 13.6 and 30.6 / 35.9;
+        // 64 rows 18.1 / 16.1 and 38.5 / 39.8, 31.1 / 35.9 at 40,001 (8,000 columns: 17.2 / 12.8)
+        if (P.N >= (RT <= 2 ? 16000 : 36000)) {
+            PGemmArgs pa{};
+            pa.N = P.N; pa.rows = rows; pa.W = P.W; pa.csum = P.csum; pa.we = P.e; pa.bias = P.b;
+            pa.planes = planes; pa.rowinfo = rowinfo; pa.Y = (i64*)pile;
+            const dim3 grid((unsigned)((P.ntiles + 3) / 4 + 7) / 8 * 8);
+            launch(timed, "plate.head_rows", k_pgemm<768, EPI_PILE, RT <= 2 ? 2 : 4, 4, 2, 2, 2>, grid, dim3(256), 0, s, pa);
+        } else if (P.N > 3072) {
             launch(timed, "plate.head_rows", k_head_rows<RT, EPI_PILE>, dim3(head_rows_grid(P.ntiles)), dim3(256), 0, s, ga);
-        else                  // layer-shaped plates: one column tile per block, K split over its four waves
+        } else                // layer-shaped plates: one column tile per block, K split over its four waves
             launch(timed, "plate.gemm", k_gemm<768, 1, 1, EPI_PILE>, dim3(P.ntiles, RT), dim3(256), 0, s, ga);
     } else {
         launch(timed, "plate.light", k_light<3072, PRO_X16, 768, 1>, dim3(rows), dim3(768), 0, s, la);

@@ -407,8 +407,9 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_pgemm(PGemmArgs a) {
 #pragma unroll
                 for (int j = 0; j < TN; j++) {
                     const unsigned col = (unsigned)(16 * (n0 + wn + j) + (lane & 15));
-                    if (row + q < a.rows && col < n)
-                        a.Y[(size_t)(row + q) * n + col] = EPI == EPI_PLAIN_ADD ? wadd(y[j][q], o[j][q]) : o[j][q];
+                    if (row + q >= a.rows || col >= n) continue;
+                    i64* to = a.Y + (size_t)(row + q) * n + col;
+                    *to = EPI == EPI_PLAIN_ADD ? wadd(y[j][q], o[j][q]) : o[j][q];
                 }
         }
     }
