@@ -700,7 +700,10 @@ static int launch_step_batched(sm_machine* m, int parts, int nrows = 0,
             GemmArgs a = gemm_args(m->mbank[l][3], nullptr, 0, nullptr, nullptr);
             a.X = m->hid; a.X32 = m->hid32; a.xstride = 3072; a.orw = m->hidor; a.rx16 = rx + 3 * 3072; a.rexls = re + 6;
             a.sfacts = m->sfacts;
-            launch(m->cfg.profile, "mproj.part", k_gemm<3072, 3, 4, EPI_PART, 192>, dim3(m->mbank[l][3].ntiles / 3 * 4, RT), dim3(256), 0, m->st, a);
+            // (column tiles a block: 192 blocks at one and two row tiles; with three a block 64 and 128, 405 / 450 against
+            // 388 / 442 us a step at 4 / 24 streams)
+            constexpr int NB = RT < 3 ? RT : 3;
+            launch(m->cfg.profile, "mproj.part", k_gemm<3072, NB, 4, EPI_PART, 192>, dim3(m->mbank[l][3].ntiles / NB * 4, RT), dim3(256), 0, m->st, a);
         }
         const bool last = l == 11;     // the last stream update lights the head
         finish_light(m->mbank[l][3], rp + 3 * 3072, m->r_resid + (l * 2 + 1) * 768,
@@ -1054,7 +1057,8 @@ static int launch_step_pythia_batched(sm_machine* m, int parts, int nrows = 0,
         }
         if (rowmap) {      // a prompt pass: position by position through each kernel
             launch(m->cfg.profile, "fc", k_gemm<768, 1, 1, EPI_PLAIN_EDGE>, dim3(gf, RT), dim3(256), 0, m->st, af);
-            launch(m->cfg.profile, "mproj.part", k_gemm<3072, 3, 4, EPI_PART, 192>, dim3(gm, RT), dim3(256), 0, m->st, am);
+            constexpr int NB = RT < 3 ? RT : 3;     // (as launch_step_batched)
+            launch(m->cfg.profile, "mproj.part", k_gemm<3072, NB, 4, EPI_PART, 192>, dim3(m->mbank[l][3].ntiles / NB * 4, RT), dim3(256), 0, m->st, am);
             launch(m->cfg.profile, "kv_rows", k_kv_rows<1>, dim3(12, B), dim3(128), 0, m->st, at);
             attend_rows<1>(m, B, at);
         }
