@@ -1254,7 +1254,12 @@ static void pgemm(sm_machine* m, const char* name, const MfmaPlate& P, int set, 
     a.planes = m->pw.pl[set]; a.rowinfo = m->pw.ri[set]; a.Y = Y; a.y = y; a.tb = m->T.tb();
     a.err = m->kind == 1 ? m->ctl + CTL_ERR : nullptr;
     const int grid = ((P.ntiles + 3) / 4) * ((rows + 63) / 64);
-    launch(m->cfg.profile, name, k_pgemm<K, EPI, 4, 4, 2, 2, 2>, dim3((grid + 7) / 8 * 8), dim3(256), 0, m->st, a);
+    // (3072 inputs: two groups of waves a block up to 300 blocks, about 1,600 rows; at 344 / 999 / 1,984 / 4,028 rows
+    // 19.3 / 21.1 / 46 / 66 us against 25.4 / 26.7 / 47 / 60)
+    if (K == 3072 && grid <= 300)
+        launch(m->cfg.profile, name, k_pgemm<K, EPI, 4, 4, 2, 2, 2, K == 3072 ? 2 : 1>, dim3((grid + 7) / 8 * 8), dim3(512), 0, m->st, a);
+    else
+        launch(m->cfg.profile, name, k_pgemm<K, EPI, 4, 4, 2, 2, 2>, dim3((grid + 7) / 8 * 8), dim3(256), 0, m->st, a);
 }
 template <int MODEL>
 static int launch_prompt(sm_machine* m, int s0, int S, int pa, int pb, const int* map) {

@@ -174,7 +174,8 @@ __global__ __launch_bounds__(512) void k_plight(PLightArgs a) {
 // TM x TN tiles, three int32 accumulators a tile (HH, MID, LL of the pile identity in sm_batch.hip); a 64-k step's
 // operands (1 KB a tile and plane) go through two LDS buffers, D steps ahead in registers.  All operands lie in memory
 // in MFMA order, so every global load and LDS access is a whole wave's consecutive 1 KB.  Blocks are numbered so that
-// each XCD (block index % 8) works on a contiguous run of row tiles.
+// each XCD (block index % 8) works on a contiguous run of row tiles.  KW = 2: two groups of such waves, each every
+// second k step, whose sums meet in LDS (half the chain of a 3072-wide bank with few blocks).
 // The machine's tiles are 64 x 64 (four waves of 32 x 32, 126 registers, four blocks a CU): at 999 / 4,028 rows fc
 // takes 23.4 / 73 us and mproj 26.5 / 59 us (0.7-1.3 POP/s of int8).  128 x 64 tiles measured 28.8 / 79 and 35.9 / 69
 // us, 128 x 128 of eight waves 26.8 / 77 and 44.6 / 69, 128 x 128 of four waves 39 / 111 and 67 / 100 (fewer blocks to
@@ -188,19 +189,20 @@ struct PGemmArgs {
     Tables tb;
     int* err;                     // the Pythia machine: its rshift assert sets SM_ERR_RANGE here
 };
-template <int K, int EPI, int MT, int NT, int WM, int WN, int D>
-__global__ __launch_bounds__(64 * WM * WN, 2) void k_pgemm(PGemmArgs a) {
+template <int K, int EPI, int MT, int NT, int WM, int WN, int D, int KW = 1>
+__global__ __launch_bounds__(64 * WM * WN * KW, 2) void k_pgemm(PGemmArgs a) {
     constexpr int KS = K / 64, CH = (MT + NT) * 2, NV = WM * WN, PER = CH / NV, TM = MT / WM, TN = NT / WN;
     constexpr bool GAUGED = EPI == EPI_GAUGED || EPI == EPI_GAUGED_EDGE, EDGE = EPI == EPI_GAUGED_EDGE || EPI == EPI_PLAIN_EDGE;
     constexpr bool PLAIN = EPI == EPI_PLAIN || EPI == EPI_PLAIN_EDGE || EPI == EPI_PLAIN_ADD;
     constexpr bool ROWS = GAUGED || EPI == EPI_PLAIN || EPI == EPI_PLAIN_EDGE;      // the outputs go to a PRow
-    static_assert(CH % NV == 0 && KS % D == 0 && D % 2 == 0, "whole chunks a wave, whole rounds of the ring");
+    static_assert(CH % NV == 0 && KS % (D * KW) == 0 && D % 2 == 0, "whole chunks a wave, whole rounds of the ring");
     static_assert(!ROWS || TN * 16 % PSW == 0, "a wave's columns are whole strips");
-    __shared__ v4p buf[2][CH][64];
+    __shared__ v4p buf[2 * KW][CH][64];
+    static_assert(KW == 1 || NV * TM * TN * 3 <= 2 * KW * CH, "the groups' accumulators meet in buf");
     __shared__ i64 rcC[16 * MT];             // a row's pile constant
     __shared__ int rcS[16 * MT], rcE[16 * MT], rcN[16 * MT];   // its power's row part and factor, n32768
     __shared__ int any32;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = (tid >> 6) % NV, kg = (tid >> 6) / NV;
     const int ntiles = (a.N + 15) / 16, nb = (ntiles + NT - 1) / NT, mb = (a.rows + 16 * MT - 1) / (16 * MT), total = nb * mb;
     // block b of XCD b % 8: the (b / 8)-th of that XCD's run of `per` tiles
     const int per = (total + 7) / 8, id = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
@@ -222,7 +224,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_pgemm(PGemmArgs a) {
 #pragma unroll
     for (int d = 0; d < D; d++)
 #pragma unroll
-        for (int i = 0; i < PER; i++) r[d][i] = src[i][d * step(i)];
+        for (int i = 0; i < PER; i++) r[d][i] = src[i][(d * KW + kg) * step(i)];
     // the rows' facts (ex, LS lo, LS hi, e2, SXh, SXl, n32768; gauged lights carry LS and its power factor)
     if (tid == 0) any32 = 0;
     __syncthreads();
@@ -252,14 +254,14 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_pgemm(PGemmArgs a) {
 #pragma unroll
         for (int j = 0; j < TN; j++) acc[i][j][0] = acc[i][j][1] = acc[i][j][2] = v4p{0, 0, 0, 0};
 #pragma unroll 1
-    for (int s0 = 0; s0 < KS; s0 += D) {
+    for (int s0 = 0; s0 < KS / KW; s0 += D) {
 #pragma unroll
         for (int d = 0; d < D; d++) {
-            v4p(*bs)[64] = buf[d & 1];
+            v4p(*bs)[64] = buf[2 * kg + (d & 1)];
 #pragma unroll
             for (int i = 0; i < PER; i++) bs[wave + NV * i][lane] = r[d][i];
             // D steps on (past the end the last step again: no branch around the loads)
-            const int nx = min(s0 + d + D, KS - 1);
+            const int nx = min(s0 + d + D, KS / KW - 1) * KW + kg;
 #pragma unroll
             for (int i = 0; i < PER; i++) r[d][i] = src[i][nx * step(i)];
             __syncthreads();
@@ -281,6 +283,25 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_pgemm(PGemmArgs a) {
                 }
             }
         }
+    }
+    if constexpr (KW > 1) {               // the second group's sums to the first
+        __syncthreads();
+        v4p* x = &buf[0][0][0] + wave * TM * TN * 3 * 64 + lane;
+        if (kg > 0)
+#pragma unroll
+            for (int i = 0; i < TM; i++)
+#pragma unroll
+                for (int j = 0; j < TN; j++)
+#pragma unroll
+                    for (int k = 0; k < 3; k++) x[((i * TN + j) * 3 + k) * 64] = acc[i][j][k];
+        __syncthreads();
+        if (kg > 0) return;
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int j = 0; j < TN; j++)
+#pragma unroll
+                for (int k = 0; k < 3; k++) acc[i][j][k] += x[((i * TN + j) * 3 + k) * 64];
     }
     // (rare) a light of +32768 among the block's rows, held as 32767: those rows' correction plane times the plate
     if (any32) {
