@@ -750,7 +750,8 @@ __global__ __launch_bounds__(256) void k_gemm(GemmArgs a) { gemm_block<K, NB, KS
 // block coordinates its own launch would give it (gx: its grid's x extent); a block's branch is uniform, so each
 // body's barriers stay block-wide, and each body keeps its own LDS.
 //   k_gemm_pair: two 768-input banks (fc with its edge, qkv), both lit by the same row kernel
-//   k_attend_mproj: the attention (one block a head and stream, 256 threads) and mproj's K-slice partials
+//   k_attend_mproj: the attention (one block a head and stream, 256 threads) and mproj's K-slice partials (NB column
+//   tiles a block)
 template <int EA, int EB>
 __global__ __launch_bounds__(256) void k_gemm_pair(GemmArgs a, GemmArgs b, int na, int gxa, int gxb) {
     const int i = blockIdx.x;
@@ -761,14 +762,14 @@ __global__ __launch_bounds__(256) void k_gemm_pair(GemmArgs a, GemmArgs b, int n
         gemm_block<768, 1, 1, EB>(b, j % gxb, j / gxb);
     }
 }
-template <int MODEL, int ARRF>
+template <int MODEL, int ARRF, int NB>
 __global__ __launch_bounds__(256) void k_attend_mproj(AttArgs a, GemmArgs b, int na, int gxb) {
     const int i = blockIdx.x;
     if (i < na) {
         attend_block<MODEL, 0, 1, 0, 256, ARRF>(a, i % 12, i / 12);
     } else {
         const int j = i - na;
-        gemm_block<3072, 3, 4, EPI_PART, 192>(b, j % gxb, j / gxb);
+        gemm_block<3072, NB, 4, EPI_PART, 192>(b, j % gxb, j / gxb);
     }
 }
 

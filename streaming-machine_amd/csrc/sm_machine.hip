@@ -1029,18 +1029,27 @@ static int launch_step_pythia_batched(sm_machine* m, int parts, int nrows = 0,
             at.cosT = m->cosT; at.sinT = m->sinT; at.rot = m->rot; at.half = m->half; at.ehalf = m->ehalf;
             at.out_or = m->attor; at.out32 = m->att32;
         }
-        const int gq = m->mbank[l][0].ntiles, gf = m->mbank[l][2].ntiles, gm = m->mbank[l][3].ntiles / 3 * 4;
+        const int gq = m->mbank[l][0].ntiles, gf = m->mbank[l][2].ntiles;
         if (!rowmap) {
             // a decode step: the two halves of the layer share launches (fc with qkv, then mproj's partials with
             // the attention), four launches a layer with proj and the row kernel
             launch(m->cfg.profile, "fc+qkv", k_gemm_pair<EPI_PLAIN_EDGE, EPI_PLAIN>, dim3(gf * RT + gq * RT), dim3(256), 0,
                    m->st, af, aq, gf * RT, gf, gq);
-            if (m->T.verified)
-                launch(m->cfg.profile, "attend+mproj.part", k_attend_mproj<1, 1>, dim3(12 * B + gm * RT), dim3(256),
-                       (size_t)m->ctx * 12, m->st, at, am, 12 * B, gm);
-            else
-                launch(m->cfg.profile, "attend+mproj.part", k_attend_mproj<1, 0>, dim3(12 * B + gm * RT), dim3(256),
-                       (size_t)m->ctx * 12, m->st, at, am, 12 * B, gm);
+            // mproj's column tiles a block: three, or RT at one and two row tiles, 192 blocks, while those and the
+            // attention's fit two blocks a CU (2 streams 276 against 285 us a step, 24 streams 322 against 333; at 32
+            // streams, 576 blocks, 362 against 338)
+            auto pair = [&](auto nb) {
+                constexpr int NB = decltype(nb)::value;
+                const int gm = m->mbank[l][3].ntiles / NB * 4;
+                if (m->T.verified)
+                    launch(m->cfg.profile, "attend+mproj.part", k_attend_mproj<1, 1, NB>, dim3(12 * B + gm * RT), dim3(256),
+                           (size_t)m->ctx * 12, m->st, at, am, 12 * B, gm);
+                else
+                    launch(m->cfg.profile, "attend+mproj.part", k_attend_mproj<1, 0, NB>, dim3(12 * B + gm * RT), dim3(256),
+                           (size_t)m->ctx * 12, m->st, at, am, 12 * B, gm);
+            };
+            if (RT < 3 && 12 * B + 192 <= 512) pair(std::integral_constant<int, RT < 3 ? RT : 3>{});
+            else pair(std::integral_constant<int, 3>{});
         } else {
             launch(m->cfg.profile, "qkv", k_gemm<768, 1, 1, EPI_PLAIN>, dim3(gq, RT), dim3(256), 0, m->st, aq);
         }
