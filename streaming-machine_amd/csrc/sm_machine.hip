@@ -280,15 +280,17 @@ struct sm_tables {
     int alen = 0;
     i64 log768 = 0, eps40 = 0;
     int verified = 0;         // every entry equals its defining formula (checked on the device at create)
-    int* scratch = nullptr;   // [1] error bits, [4..7] mismatch counts
+    int* scratch = nullptr;   // [4..7] mismatch counts
     int* posn = nullptr;      // [SM_STAGE_ATT_CTX] the numbers 0, 1, ..: the attention entry points' positions
-    int* herr = nullptr;      // pinned host memory: their error bits
+    int* herr = nullptr;      // pinned host memory, SM_ERR_SLOTS lines: a call's error word
+    mutable unsigned next = 0;   // (a call takes the next line, so that calls on several threads each have their own)
     // sm_stage_attend_split's score row, chunk maxima and accumulators (made at its first call, for ctx <= 8192)
     i64 *asc = nullptr, *acm = nullptr, *aacc = nullptr;
     Tables tb() const { return Tables{LOG2, EXP2, PHI, ARR, alen, log768, eps40, GPOW, HPOW, PGPOW}; }
 };
 
 #define SM_STAGE_ATT_CTX 8192      // positions of the attention entry points
+#define SM_ERR_SLOTS 256           // their error words, 64 bytes apart
 static int upload_table(int** dst, const i64* src, size_t n, i64 lo, i64 hi, const char* name) {
     std::vector<int> v(n);
     for (size_t i = 0; i < n; i++) {
@@ -330,7 +332,7 @@ static int tables_init(sm_tables& T, const i64* phi, const i64* arr, int alen, c
         for (int i = 0; i < SM_STAGE_ATT_CTX; i++) n[i] = i;
         if ((rc = dalloc(&T.posn, n.size()))) return rc;
         HIP_TRY(hipMemcpy(T.posn, n.data(), n.size() * 4, hipMemcpyHostToDevice));
-        if (hipHostMalloc(&T.herr, 64, hipHostMallocDefault) != hipSuccess) {
+        if (hipHostMalloc(&T.herr, SM_ERR_SLOTS * 64, hipHostMallocDefault) != hipSuccess) {
             T.herr = nullptr;
             return fail(SM_E_OOM, "hipHostMalloc: the error word");
         }
@@ -2073,17 +2075,18 @@ extern "C" int sm_stage_race(const int64_t* v, int64_t n, int64_t* out_index, vo
     HIP_TRY(hipGetLastError());
     return SM_OK;
 }
-// The attention entry points' end: the launched kernels done, and the error they report.  A call is its launches, one
-// copy of the error word into pinned memory and one wait: the position is an entry of a device array of numbers (a
-// copy and a wait of its own before the launch, and the error word into pageable memory, made a call of 9 us of
-// kernels take 47 us).
-static int stage_attend_end(const sm_tables* t, hipStream_t s, const char* what) {
-    HIP_TRY(hipMemcpyAsync(t->herr, t->scratch + 1, 4, hipMemcpyDeviceToHost, s));
+// The attention entry points' error word: a line of pinned host memory that the kernels store to (a value past 32
+// bits), so a call is its launches and one wait.  (The position is an entry of a device array of numbers.  With a copy
+// and a wait for the position before the launch and the error word copied into pageable memory, a call of 9 us of
+// kernels took 47 us; with the error word copied into pinned memory 25 us.)
+static int* stage_err(const sm_tables* t) {
+    int* w = t->herr + __atomic_fetch_add(&t->next, 1u, __ATOMIC_RELAXED) % SM_ERR_SLOTS * 16;
+    *static_cast<volatile int*>(w) = 0;
+    return w;
+}
+static int stage_attend_end(const int* herr, hipStream_t s, const char* what) {
     HIP_TRY(hipStreamSynchronize(s));
-    if (*static_cast<volatile int*>(t->herr) & SM_ERR_V32) {
-        HIP_TRY(hipMemset(t->scratch + 1, 0, 4));
-        return fail(SM_E_OVERFLOW, what);
-    }
+    if (*static_cast<const volatile int*>(herr) & SM_ERR_V32) return fail(SM_E_OVERFLOW, what);
     return SM_OK;
 }
 extern "C" int sm_stage_attend(const sm_tables* t, const int64_t* qkv, int16_t* k16, int64_t* km, int32_t* ek, int32_t* v,
@@ -2093,10 +2096,10 @@ extern "C" int sm_stage_attend(const sm_tables* t, const int64_t* qkv, int16_t* 
     hipStream_t s = (hipStream_t)stream;
     AttArgs a{};
     a.QKV = (const i64*)qkv; a.K16 = k16; a.KM = (i64*)km; a.EK = ek; a.V = v; a.out = (i64*)out; a.pos = t->posn + pos; a.ctx = ctx;
-    a.tb = t->tb(); a.err = t->scratch + 1;
+    a.tb = t->tb(); a.herr = stage_err(t);
     launch(g_kt.stages, "stage.attend", k_attend<0, 1, 0>, dim3(12, 1), dim3(NTHR), (size_t)ctx * 12, s, a);
     HIP_TRY(hipGetLastError());
-    return stage_attend_end(t, s, "sm_stage_attend: a value left 32 bits");
+    return stage_attend_end(a.herr, s, "sm_stage_attend: a value left 32 bits");
 }
 
 // the same attention spread over chunks of 64 positions, the batch-1 machine's kernels for positions from its split
@@ -2119,7 +2122,7 @@ extern "C" int sm_stage_attend_split(const sm_tables* t, const int64_t* qkv, int
     hipStream_t s = (hipStream_t)stream;
     AttArgs a{};
     a.QKV = (const i64*)qkv; a.K16 = k16; a.KM = (i64*)km; a.EK = ek; a.V = v; a.out = (i64*)out; a.pos = t->posn + pos; a.ctx = ctx;
-    a.tb = t->tb(); a.err = t->scratch + 1;
+    a.tb = t->tb(); a.herr = stage_err(t);
     a.asc = tt->asc; a.acm = tt->acm; a.aacc = tt->aacc; a.ncm = ncm;
     const dim3 grid(12, (ctx + ACH_SPLIT - 1) / ACH_SPLIT);
     const bool timed = g_kt.stages;
@@ -2127,7 +2130,7 @@ extern "C" int sm_stage_attend_split(const sm_tables* t, const int64_t* qkv, int
     launch(timed, "stage.attend.mix", k_att_mix<0, 0>, grid, dim3(256), 0, s, a);
     launch(timed, "stage.attend.finish", k_att_finish<0, 0>, dim3(12), dim3(64), 0, s, a);
     HIP_TRY(hipGetLastError());
-    return stage_attend_end(t, s, "sm_stage_attend_split: a value left 32 bits");
+    return stage_attend_end(a.herr, s, "sm_stage_attend_split: a value left 32 bits");
 }
 
 extern "C" int sm_stage_attend_rows(const sm_tables* t, const int64_t* qkv, int32_t rows, int16_t* k16, int64_t* km,
@@ -2138,10 +2141,10 @@ extern "C" int sm_stage_attend_rows(const sm_tables* t, const int64_t* qkv, int3
     hipStream_t s = (hipStream_t)stream;
     AttArgs a{};
     a.QKV = (const i64*)qkv; a.K16 = k16; a.KM = (i64*)km; a.EK = ek; a.V = v; a.out = (i64*)out; a.pos = t->posn + pos; a.ctx = ctx;
-    a.tb = t->tb(); a.err = t->scratch + 1;
+    a.tb = t->tb(); a.herr = stage_err(t);
     launch(g_kt.stages, "stage.attend_rows", k_attend<0, 0, 1>, dim3(12, rows), dim3(NTHR), (size_t)ctx * 12, s, a);      // the batched machine's kernel
     HIP_TRY(hipGetLastError());
-    return stage_attend_end(t, s, "sm_stage_attend_rows: a value left 32 bits");
+    return stage_attend_end(a.herr, s, "sm_stage_attend_rows: a value left 32 bits");
 }
 
 // tile_cols > 0: a GEMV plate (one light row per product); tile_cols == 0: an MFMA plate (rows of lights) with
