@@ -1666,27 +1666,28 @@ __global__ __launch_bounds__(NTHR) void k_stage_rows(const i64* X, int n, int ga
 // time before it looks at any (a value a trip of the loop waits a memory latency each: 50,257 values took 19.7 us).
 // MANY = 0: one block, which writes its winner.  MANY = 1: blocks in a grid stride, each then putting its winner into
 // *out where it beats the one that is there (*out is -1 on entry, k_race_none): no scratch, so calls on any streams
-// are independent.  Back to back, one block / many: 8,192 values 5.2 / 5.8 us, 16,000 6.3 / 6.2, 50,257 11.5 / 6.7,
+// are independent.  Up to 8,192 values the one block takes one a trip (V = 1: 1,111 values 4.27 us against 4.99 with
+// eight, 8,000 5.37 / 5.27).  Back to back, one block / many: 8,192 values 5.2 / 5.8 us, 16,000 6.3 / 6.2, 50,257 11.5 / 6.7,
 // 200,000 34.7 / 8.2, 3,000,000 457 / 13.3; many blocks of 256 threads up to 131,072 values (50,257: 6.7 us, 7.3 at 512
 // threads, 8.5 at 1024), of 512 past that (3,000,000: 13.3 against 16.0 us).
 #define RACE_V 8
 __global__ void k_race_none(i64* out) { *out = -1; }
-template <int MANY, int NT>
+template <int MANY, int NT, int V = RACE_V>
 __global__ __launch_bounds__(NT) void k_stage_race(const i64* v, i64 n, i64* out) {
     constexpr int NW = NT / 64;
     __shared__ i64 bvs[NW];
     __shared__ i64 bis[NW];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     i64 bv = 0, bi = -1;
-    for (i64 b = (i64)blockIdx.x * (NT * RACE_V); b < n; b += (i64)gridDim.x * (NT * RACE_V)) {
-        i64 x[RACE_V];
+    for (i64 b = (i64)blockIdx.x * (NT * V); b < n; b += (i64)gridDim.x * (NT * V)) {
+        i64 x[V];
 #pragma unroll
-        for (int k = 0; k < RACE_V; k++) {
+        for (int k = 0; k < V; k++) {
             const i64 i = b + tid + NT * k;
             x[k] = v[i < n ? i : n - 1];
         }
 #pragma unroll
-        for (int k = 0; k < RACE_V; k++) {
+        for (int k = 0; k < V; k++) {
             const i64 i = b + tid + NT * k;                 // (grows: a later equal value never wins)
             if (i < n && (bi < 0 || x[k] > bv)) { bv = x[k]; bi = i; }
         }

@@ -2082,7 +2082,9 @@ extern "C" int sm_stage_race(const int64_t* v, int64_t n, int64_t* out_index, vo
     if (n <= 0 || !v || !out_index) return fail(SM_E_ARG, "sm_stage_race: arguments");
     hipStream_t s = (hipStream_t)stream;
     // (an index written over the values themselves is raced by one block, which writes after it has read them)
-    if (n <= SM_RACE_ONE || (out_index >= v && out_index < v + n)) {
+    if (n <= 8192) {
+        launch(g_kt.stages, "stage.race", k_stage_race<0, 1024, 1>, dim3(1), dim3(1024), 0, s, (const i64*)v, n, (i64*)out_index);
+    } else if (n <= SM_RACE_ONE || (out_index >= v && out_index < v + n)) {
         launch(g_kt.stages, "stage.race", k_stage_race<0, 1024>, dim3(1), dim3(1024), 0, s, (const i64*)v, n, (i64*)out_index);
     } else {
         launch(g_kt.stages, "stage.race.none", k_race_none, dim3(1), dim3(1), 0, s, (i64*)out_index);
