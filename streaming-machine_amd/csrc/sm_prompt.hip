@@ -8,8 +8,8 @@
 //   k_pattend   attention (base2.py:94-99) of 16 query positions a block, scores and value sums by MFMA
 //   k_plight    the rows' lights (base2.py:24-27, 55-60); the Pythia machine's two gauges are k_py_rows'
 // Why: in passes of 64 rows each launch (5-9 us, latency-bound) serves 64 rows, and the attention, one block a (head,
-// row), reads a row's whole cache for one query.  Same box, a whole call: GPT-2, one 1000-word prompt 9.42 -> 2.27 ms;
-// 19 prompts of 213 words and 17 words each 39.1 -> 12.3 ms; 64 prompts of 32 words and 128 words 85.5 -> 73.4 ms.
+// row), reads a row's whole cache for one query.  Same box, a whole call: GPT-2, one 1000-word prompt 9.40 -> 2.14 ms;
+// 19 prompts of 213 words and 17 words each 39.2 -> 12.4 ms; 64 prompts of 32 words and 128 words 85.8 -> 73.0 ms.
 #include "sm_kernels.h"
 #include <cstddef>
 #include <type_traits>
@@ -177,7 +177,7 @@ __global__ __launch_bounds__(512) void k_plight(PLightArgs a) {
 // each XCD (block index % 8) works on a contiguous run of row tiles.  KW = 2: two groups of such waves, each every
 // second k step, whose sums meet in LDS (half the chain of a 3072-wide bank with few blocks).
 // The machine's tiles are 64 x 64 (four waves of 32 x 32, 126 registers, four blocks a CU): at 999 / 4,028 rows fc
-// takes 23.4 / 73 us and mproj 26.5 / 59 us (0.7-1.3 POP/s of int8).  128 x 64 tiles measured 28.8 / 79 and 35.9 / 69
+// takes 23.4 / 73 us and mproj 26.5 / 59 us with one group (0.7-1.3 POP/s of int8).  128 x 64 tiles measured 28.8 / 79 and 35.9 / 69
 // us, 128 x 128 of eight waves 26.8 / 77 and 44.6 / 69, 128 x 128 of four waves 39 / 111 and 67 / 100 (fewer blocks to
 // run beside each other's barriers and epilogues), four steps ahead in place of two 24.4 / 78 and 23.0 / 57.
 struct PGemmArgs {
