@@ -170,7 +170,6 @@ struct AttArgs {
     int ctx;
     Tables tb;
     int* err;           // bit 0: a value left 32 bits with no V64 to hold it; bit 1: a value the reference asserts on
-    int* herr;          // (when non-null) host memory: SM_ERR_V32 is stored there instead (the stage entry points)
     const int* rec_pos; i64* ratt;
     // the Pythia machine: turns on the first rot dims of q and k, the scores' half-log2(head size)
     const int* cosT; const int* sinT;   // [npos][rot / 2] at 2^-30

@@ -980,8 +980,7 @@ SMD void v_store(const AttArgs& a, size_t hrow, int p, int lane, i64 x) {
             if (wide) atomicOr(a.vbig + hrow, 1);
         }
     } else if (wide && lane == 0) {
-        if (a.herr) *a.herr = SM_ERR_V32;
-        else atomicOr(a.err, SM_ERR_V32);
+        *a.err = SM_ERR_V32;                                // (the stage entry points: a word of host memory)
     }
 }
 // The (stream, head)'s mark of values past 32 bits (vbig), as a vector load issued with the cached rows and waited

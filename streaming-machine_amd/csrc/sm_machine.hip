@@ -2117,10 +2117,10 @@ extern "C" int sm_stage_attend(const sm_tables* t, const int64_t* qkv, int16_t* 
     hipStream_t s = (hipStream_t)stream;
     AttArgs a{};
     a.QKV = (const i64*)qkv; a.K16 = k16; a.KM = (i64*)km; a.EK = ek; a.V = v; a.out = (i64*)out; a.pos = t->posn + pos; a.ctx = ctx;
-    a.tb = t->tb(); a.herr = stage_err(t);
+    a.tb = t->tb(); a.err = stage_err(t);
     launch(g_kt.stages, "stage.attend", k_attend<0, 1, 0>, dim3(12, 1), dim3(NTHR), (size_t)ctx * 12, s, a);
     HIP_TRY(hipGetLastError());
-    return stage_attend_end(a.herr, s, "sm_stage_attend: a value left 32 bits");
+    return stage_attend_end(a.err, s, "sm_stage_attend: a value left 32 bits");
 }
 
 // the same attention spread over chunks of 64 positions, the batch-1 machine's kernels for positions from its split
@@ -2143,7 +2143,7 @@ extern "C" int sm_stage_attend_split(const sm_tables* t, const int64_t* qkv, int
     hipStream_t s = (hipStream_t)stream;
     AttArgs a{};
     a.QKV = (const i64*)qkv; a.K16 = k16; a.KM = (i64*)km; a.EK = ek; a.V = v; a.out = (i64*)out; a.pos = t->posn + pos; a.ctx = ctx;
-    a.tb = t->tb(); a.herr = stage_err(t);
+    a.tb = t->tb(); a.err = stage_err(t);
     a.asc = tt->asc; a.acm = tt->acm; a.aacc = tt->aacc; a.ncm = ncm;
     const dim3 grid(12, (ctx + ACH_SPLIT - 1) / ACH_SPLIT);
     const bool timed = g_kt.stages;
@@ -2151,7 +2151,7 @@ extern "C" int sm_stage_attend_split(const sm_tables* t, const int64_t* qkv, int
     launch(timed, "stage.attend.mix", k_att_mix<0, 0>, grid, dim3(256), 0, s, a);
     launch(timed, "stage.attend.finish", k_att_finish<0, 0>, dim3(12), dim3(64), 0, s, a);
     HIP_TRY(hipGetLastError());
-    return stage_attend_end(a.herr, s, "sm_stage_attend_split: a value left 32 bits");
+    return stage_attend_end(a.err, s, "sm_stage_attend_split: a value left 32 bits");
 }
 
 extern "C" int sm_stage_attend_rows(const sm_tables* t, const int64_t* qkv, int32_t rows, int16_t* k16, int64_t* km,
@@ -2162,10 +2162,10 @@ extern "C" int sm_stage_attend_rows(const sm_tables* t, const int64_t* qkv, int3
     hipStream_t s = (hipStream_t)stream;
     AttArgs a{};
     a.QKV = (const i64*)qkv; a.K16 = k16; a.KM = (i64*)km; a.EK = ek; a.V = v; a.out = (i64*)out; a.pos = t->posn + pos; a.ctx = ctx;
-    a.tb = t->tb(); a.herr = stage_err(t);
+    a.tb = t->tb(); a.err = stage_err(t);
     launch(g_kt.stages, "stage.attend_rows", k_attend<0, 0, 1>, dim3(12, rows), dim3(NTHR), (size_t)ctx * 12, s, a);      // the batched machine's kernel
     HIP_TRY(hipGetLastError());
-    return stage_attend_end(a.herr, s, "sm_stage_attend_rows: a value left 32 bits");
+    return stage_attend_end(a.err, s, "sm_stage_attend_rows: a value left 32 bits");
 }
 
 // tile_cols > 0: a GEMV plate (one light row per product); tile_cols == 0: an MFMA plate (rows of lights) with
