@@ -202,7 +202,8 @@ int sm_stage_attend(const sm_tables* t, const int64_t* qkv, int16_t* k16, int64_
 /* The same attention as sm_stage_attend (the same arguments, caches and results), spread over the GPU as the batch-1
  * machine runs it from its att_split position on: each head's positions in chunks of 64, one block a chunk, three
  * launches (scores and chunk maxima; arrivals against the head's maximum with the value sums added exactly; the
- * divisor).  ctx at most 8192; the first call allocates its scratch (score row, chunk maxima, sums) with the tables. */
+ * divisor).  ctx at most 8192; the first call allocates its scratch (score row, chunk maxima, sums) with the tables;
+ * calls that share tables take turns on it. */
 int sm_stage_attend_split(const sm_tables* t, const int64_t* qkv, int16_t* k16, int64_t* km, int32_t* ek, int32_t* v,
                           int32_t pos, int32_t ctx, int64_t* out, void* stream);
 

@@ -284,7 +284,9 @@ struct sm_tables {
     int* posn = nullptr;      // [SM_STAGE_ATT_CTX] the numbers 0, 1, ..: the attention entry points' positions
     int* herr = nullptr;      // pinned host memory, SM_ERR_SLOTS lines: a call's error word
     mutable unsigned next = 0;   // (a call takes the next line, so that calls on several threads each have their own)
-    // sm_stage_attend_split's score row, chunk maxima and accumulators (made at its first call, for ctx <= 8192)
+    // sm_stage_attend_split's score row, chunk maxima and accumulators (made at its first call, for ctx <= 8192), one
+    // set: a call holds the lock from there to its wait, so that calls on several threads or streams take turns
+    mutable std::mutex split_mu;
     i64 *asc = nullptr, *acm = nullptr, *aacc = nullptr;
     Tables tb() const { return Tables{LOG2, EXP2, PHI, ARR, alen, log768, eps40, GPOW, HPOW, PGPOW}; }
 };
@@ -352,7 +354,6 @@ static void tables_free(sm_tables& T) {
     hfree(T.LOG2); hfree(T.EXP2); hfree(T.PHI); hfree(T.ARR); hfree(T.GPOW); hfree(T.HPOW); hfree(T.PGPOW); hfree(T.scratch);
     hfree(T.asc); hfree(T.acm); hfree(T.aacc); hfree(T.posn);
     if (T.herr) (void)hipHostFree(T.herr);
-    T = sm_tables();
 }
 
 // ---------------------------------------------------------------------------------------------------------
@@ -2129,6 +2130,7 @@ extern "C" int sm_stage_attend_split(const sm_tables* t, const int64_t* qkv, int
                                      int32_t* v, int32_t pos, int32_t ctx, int64_t* out, void* stream) {
     if (!t || !qkv || !k16 || !km || !ek || !v || !out || ctx <= 0 || pos < 0 || pos >= ctx || ctx > SM_STAGE_ATT_CTX)
         return fail(SM_E_ARG, "sm_stage_attend_split: arguments");
+    std::lock_guard<std::mutex> lock(t->split_mu);
     sm_tables* tt = const_cast<sm_tables*>(t);
     const int ncm = (SM_STAGE_ATT_CTX + ACH_SPLIT - 1) / ACH_SPLIT;
     if (!tt->asc) {

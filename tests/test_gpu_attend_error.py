@@ -51,3 +51,40 @@ def test_threads(sm):
     [x.join() for x in ths]
     assert got == {0: [0] * 300, 1: [-6] * 300}
     t.close()
+
+
+@pytest.mark.parametrize("fn", ["attend", "attend_split", "attend_rows"])
+def test_threads_rows(sm, fn):
+    """three threads, each on its own stream with its own caches at a position past several chunks, with the same
+    tables: every call gives the row that the same call gives alone (attend_split's scratch belongs to the tables)"""
+    t = sm.Tables(sm.tables())
+    rows = 3 if fn == "attend_rows" else 1
+    jobs = []
+    for k in range(3):
+        g = torch.Generator(device="cuda")
+        g.manual_seed(70 + k)
+        n = lambda *s: (torch.randn(s, generator=g, device="cuda", dtype=torch.float64) * 65536).round()      # noqa: E731
+        pos = (130, 199, 255)[k]
+        c = [n(rows, 12, CTX, 64).clamp(-32768, 32767).to(torch.int16), torch.zeros((rows, 12, CTX), dtype=torch.int64, device="cuda"),
+             torch.full((rows, 12, CTX), -13, dtype=torch.int32, device="cuda"), n(rows, 12, CTX, 64).to(torch.int32)]
+        qkv, o = n(rows, 2304).to(torch.int64), torch.zeros((rows, 768), dtype=torch.int64, device="cuda")
+        args = [qkv.data_ptr()] + ([rows] if rows > 1 else []) + [x.data_ptr() for x in c] + [pos, CTX, o.data_ptr()]
+        getattr(sm.stages, fn)(t, *args)
+        torch.cuda.synchronize()
+        jobs.append((args, o, o.clone(), (c, qkv), torch.cuda.Stream()))
+    bad = []
+
+    def work(k):
+        args, o, want, _, s = jobs[k]
+        for i in range(200):
+            getattr(sm.stages, fn)(t, *args, stream=s.cuda_stream)
+            with torch.cuda.stream(s):
+                if not torch.equal(o, want):
+                    bad.append((k, i))
+                o.zero_()
+    ths = [threading.Thread(target=work, args=(k,)) for k in range(3)]
+    [x.start() for x in ths]
+    [x.join() for x in ths]
+    assert not bad, bad[:4]
+    assert any(int(w.abs().max()) > 0 for _, _, w, _, _ in jobs)
+    t.close()
