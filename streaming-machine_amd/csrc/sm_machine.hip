@@ -27,6 +27,7 @@
 #include <map>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 static thread_local std::string g_err;
@@ -274,6 +275,8 @@ static void free_mfma_plate(MfmaPlate& P) {
 
 // ---------------------------------------------------------------------------------------------------------
 // tables
+#define SM_STAGE_ATT_CTX 8192      // positions of the attention entry points
+#define SM_ERR_SLOTS 256           // their error words, 64 bytes apart
 struct sm_tables {
     int* LOG2 = nullptr; int* EXP2 = nullptr; int* PHI = nullptr; int* ARR = nullptr;
     int* GPOW = nullptr; int* HPOW = nullptr; int* PGPOW = nullptr;
@@ -282,8 +285,9 @@ struct sm_tables {
     int verified = 0;         // every entry equals its defining formula (checked on the device at create)
     int* scratch = nullptr;   // [4..7] mismatch counts
     int* posn = nullptr;      // [SM_STAGE_ATT_CTX] the numbers 0, 1, ..: the attention entry points' positions
-    int* herr = nullptr;      // pinned host memory, SM_ERR_SLOTS lines: a call's error word
-    mutable unsigned next = 0;   // (a call takes the next line, so that calls on several threads each have their own)
+    int* herr = nullptr;      // pinned host memory, SM_ERR_SLOTS lines: a call's error word (StageErr)
+    mutable std::atomic<unsigned> next{0};                    // where a call looks for a free line
+    mutable std::atomic<bool> taken[SM_ERR_SLOTS] = {};       // the lines that calls in flight hold
     // sm_stage_attend_split's score row, chunk maxima and accumulators (made at its first call, for ctx <= 8192), one
     // set: a call holds the lock from there to its wait, so that calls on several threads or streams take turns
     mutable std::mutex split_mu;
@@ -291,8 +295,6 @@ struct sm_tables {
     Tables tb() const { return Tables{LOG2, EXP2, PHI, ARR, alen, log768, eps40, GPOW, HPOW, PGPOW}; }
 };
 
-#define SM_STAGE_ATT_CTX 8192      // positions of the attention entry points
-#define SM_ERR_SLOTS 256           // their error words, 64 bytes apart
 static int upload_table(int** dst, const i64* src, size_t n, i64 lo, i64 hi, const char* name) {
     std::vector<int> v(n);
     for (size_t i = 0; i < n; i++) {
@@ -2101,27 +2103,41 @@ extern "C" int sm_stage_race(const int64_t* v, int64_t n, int64_t* out_index, vo
 // bits), so a call is its launches and one wait.  (The position is an entry of a device array of numbers.  With a copy
 // and a wait for the position before the launch and the error word copied into pageable memory, a call of 9 us of
 // kernels took 47 us; with the error word copied into pinned memory 25 us.)
-static int* stage_err(const sm_tables* t) {
-    int* w = t->herr + __atomic_fetch_add(&t->next, 1u, __ATOMIC_RELAXED) % SM_ERR_SLOTS * 16;
-    *static_cast<volatile int*>(w) = 0;
-    return w;
-}
-static int stage_attend_end(const int* herr, hipStream_t s, const char* what) {
-    HIP_TRY(hipStreamSynchronize(s));
-    if (*static_cast<const volatile int*>(herr) & SM_ERR_V32) return fail(SM_E_OVERFLOW, what);
-    return SM_OK;
-}
+// A call holds its line from before its launches until its wait has returned: a line taken in turn alone would come
+// round again, after SM_ERR_SLOTS calls of other threads, while a call that waits behind long work on its stream still
+// has it.  With every line held (as many calls in flight) a call waits for one of them to return.
+struct StageErr {
+    const sm_tables* t;
+    unsigned i;
+    explicit StageErr(const sm_tables* tab) : t(tab) {
+        for (unsigned k = 1;; k++) {
+            i = t->next.fetch_add(1, std::memory_order_relaxed) % SM_ERR_SLOTS;
+            if (!t->taken[i].exchange(true, std::memory_order_acquire)) break;
+            if (k % SM_ERR_SLOTS == 0) std::this_thread::yield();
+        }
+        *static_cast<volatile int*>(word()) = 0;
+    }
+    ~StageErr() { t->taken[i].store(false, std::memory_order_release); }
+    StageErr(const StageErr&) = delete;
+    int* word() const { return t->herr + 16 * i; }
+    int end(hipStream_t s, const char* what) const {
+        HIP_TRY(hipStreamSynchronize(s));
+        if (*static_cast<const volatile int*>(word()) & SM_ERR_V32) return fail(SM_E_OVERFLOW, what);
+        return SM_OK;
+    }
+};
 extern "C" int sm_stage_attend(const sm_tables* t, const int64_t* qkv, int16_t* k16, int64_t* km, int32_t* ek, int32_t* v,
                                int32_t pos, int32_t ctx, int64_t* out, void* stream) {
     if (!t || !qkv || !k16 || !km || !ek || !v || !out || ctx <= 0 || pos < 0 || pos >= ctx || ctx > 8192)
         return fail(SM_E_ARG, "sm_stage_attend: arguments");
     hipStream_t s = (hipStream_t)stream;
+    const StageErr err(t);
     AttArgs a{};
     a.QKV = (const i64*)qkv; a.K16 = k16; a.KM = (i64*)km; a.EK = ek; a.V = v; a.out = (i64*)out; a.pos = t->posn + pos; a.ctx = ctx;
-    a.tb = t->tb(); a.err = stage_err(t);
+    a.tb = t->tb(); a.err = err.word();
     launch(g_kt.stages, "stage.attend", k_attend<0, 1, 0>, dim3(12, 1), dim3(NTHR), (size_t)ctx * 12, s, a);
     HIP_TRY(hipGetLastError());
-    return stage_attend_end(a.err, s, "sm_stage_attend: a value left 32 bits");
+    return err.end(s, "sm_stage_attend: a value left 32 bits");
 }
 
 // the same attention spread over chunks of 64 positions, the batch-1 machine's kernels for positions from its split
@@ -2143,9 +2159,10 @@ extern "C" int sm_stage_attend_split(const sm_tables* t, const int64_t* qkv, int
         }
     }
     hipStream_t s = (hipStream_t)stream;
+    const StageErr err(t);
     AttArgs a{};
     a.QKV = (const i64*)qkv; a.K16 = k16; a.KM = (i64*)km; a.EK = ek; a.V = v; a.out = (i64*)out; a.pos = t->posn + pos; a.ctx = ctx;
-    a.tb = t->tb(); a.err = stage_err(t);
+    a.tb = t->tb(); a.err = err.word();
     a.asc = tt->asc; a.acm = tt->acm; a.aacc = tt->aacc; a.ncm = ncm;
     const dim3 grid(12, (ctx + ACH_SPLIT - 1) / ACH_SPLIT);
     const bool timed = g_kt.stages;
@@ -2153,7 +2170,7 @@ extern "C" int sm_stage_attend_split(const sm_tables* t, const int64_t* qkv, int
     launch(timed, "stage.attend.mix", k_att_mix<0, 0>, grid, dim3(256), 0, s, a);
     launch(timed, "stage.attend.finish", k_att_finish<0, 0>, dim3(12), dim3(64), 0, s, a);
     HIP_TRY(hipGetLastError());
-    return stage_attend_end(a.err, s, "sm_stage_attend_split: a value left 32 bits");
+    return err.end(s, "sm_stage_attend_split: a value left 32 bits");
 }
 
 extern "C" int sm_stage_attend_rows(const sm_tables* t, const int64_t* qkv, int32_t rows, int16_t* k16, int64_t* km,
@@ -2162,12 +2179,13 @@ extern "C" int sm_stage_attend_rows(const sm_tables* t, const int64_t* qkv, int3
         ctx > 8192)
         return fail(SM_E_ARG, "sm_stage_attend_rows: arguments");
     hipStream_t s = (hipStream_t)stream;
+    const StageErr err(t);
     AttArgs a{};
     a.QKV = (const i64*)qkv; a.K16 = k16; a.KM = (i64*)km; a.EK = ek; a.V = v; a.out = (i64*)out; a.pos = t->posn + pos; a.ctx = ctx;
-    a.tb = t->tb(); a.err = stage_err(t);
+    a.tb = t->tb(); a.err = err.word();
     launch(g_kt.stages, "stage.attend_rows", k_attend<0, 0, 1>, dim3(12, rows), dim3(NTHR), (size_t)ctx * 12, s, a);      // the batched machine's kernel
     HIP_TRY(hipGetLastError());
-    return stage_attend_end(a.err, s, "sm_stage_attend_rows: a value left 32 bits");
+    return err.end(s, "sm_stage_attend_rows: a value left 32 bits");
 }
 
 // tile_cols > 0: a GEMV plate (one light row per product); tile_cols == 0: an MFMA plate (rows of lights) with

@@ -88,3 +88,30 @@ def test_threads_rows(sm, fn):
     assert not bad, bad[:4]
     assert any(int(w.abs().max()) > 0 for _, _, w, _, _ in jobs)
     t.close()
+
+
+def test_calls_that_wait(sm):
+    """300 calls, more than there are error words, wait behind long work on one stream, each in a thread of its own: the
+    first hundred past 32 bits report that, the others nothing"""
+    t = sm.Tables(sm.tables())
+    z = lambda dt, *s: torch.zeros(s, dtype=dt, device="cuda")      # noqa: E731
+    qs = [z(torch.int64, 2304) for _ in range(2)]
+    qs[1][1536 + 700] = 2 ** 31
+    c = (z(torch.int16, 12, CTX, 64), z(torch.int64, 12, CTX), z(torch.int32, 12, CTX), z(torch.int32, 12, CTX, 64))
+    o = z(torch.int64, 768)
+    torch.cuda.synchronize()
+    spin = torch.cuda.Stream()
+    with torch.cuda.stream(spin):
+        torch.cuda._sleep(1_000_000_000)                   # (0.4 s; the calls' launches take a few milliseconds)
+    got = [0] * 300
+
+    def work(k):
+        try:
+            sm.stages.attend(t, qs[k < 100].data_ptr(), *[x.data_ptr() for x in c], 3, CTX, o.data_ptr(), stream=spin.cuda_stream)
+        except sm.SmError as e:
+            got[k] = e.code
+    ths = [threading.Thread(target=work, args=(k,)) for k in range(300)]
+    [x.start() for x in ths]
+    [x.join() for x in ths]
+    assert got == [-6] * 100 + [0] * 200
+    t.close()
