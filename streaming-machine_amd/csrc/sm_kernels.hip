@@ -1705,8 +1705,10 @@ __global__ __launch_bounds__(NT) void k_stage_race(const i64* v, i64 n, i64* out
         if constexpr (MANY) {
             u64* o = reinterpret_cast<u64*>(out);
             u64 cur = atomicAdd(o, 0ull);
-            // (each failed exchange means that another block's winner came in: at most gridDim.x of them)
-            while ((i64)cur < 0 || bv > v[cur] || (bv == v[cur] && (u64)bi < cur)) {
+            // (each failed exchange means that another block's winner came in: at most gridDim.x of them.  An index
+            // that is no index of v, the -1 or one from a race of other values that a caller lets share the word, is
+            // replaced and never read through)
+            while (cur >= (u64)n || bv > v[cur] || (bv == v[cur] && (u64)bi < cur)) {
                 const u64 old = atomicCAS(o, cur, (u64)bi);
                 if (old == cur) break;
                 cur = old;

@@ -49,3 +49,22 @@ def test_two_streams(sm):
     torch.cuda.synchronize()
     for k in range(2):
         assert (outs[k] == int(vs[k].argmax())).all()
+
+
+def test_shared_word(sm):
+    """races of a long and a short row on two streams into one word: neither reads its own row at the other's index,
+    and a race after both has its own winner"""
+    rng = np.random.default_rng(6)
+    vs = [torch.from_numpy(rng.integers(-2 ** 40, 2 ** 40, n)).cuda() for n in (1048577, 18433)]
+    vs[0][1048576] = 2 ** 41
+    out = torch.zeros(1, dtype=torch.int64, device="cuda")
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    torch.cuda.synchronize()
+    for _ in range(100):
+        for v, s in zip(vs, streams):
+            sm.stages.race(v.data_ptr(), len(v), out.data_ptr(), stream=s.cuda_stream)
+    torch.cuda.synchronize()
+    assert 0 <= int(out[0]) < 1048577
+    sm.stages.race(vs[1].data_ptr(), len(vs[1]), out.data_ptr())
+    torch.cuda.synchronize()
+    assert int(out[0]) == int(vs[1].argmax())
