@@ -1661,14 +1661,16 @@ __global__ __launch_bounds__(NTHR) void k_stage_rows(const i64* X, int n, int ga
     }
     if (tid == 0) ex[blockIdx.x] = e;
 }
-// The race over n values: largest, ties to the lowest index (base2.py:34-40).  A thread requests RACE_V values at a
-// time before it looks at any (a value a trip of the loop waits a memory latency each: 50,257 values took 19.7 us).
+// The race over n values: largest, ties to the lowest index (base2.py:34-40).
 // MANY = 0: one block, which writes its winner.  MANY = 1: blocks in a grid stride, each then putting its winner into
 // *out where it beats the one that is there (*out is -1 on entry, k_race_none): no scratch, so calls on any streams
-// are independent.  Up to 8,192 values the one block takes one a trip (V = 1: 1,111 values 4.27 us against 4.99 with
-// eight, 8,000 5.37 / 5.27).  Back to back, one block / many: 8,192 values 5.2 / 5.8 us, 16,000 6.3 / 6.2, 50,257 11.5 / 6.7,
-// 200,000 34.7 / 8.2, 3,000,000 457 / 13.3; many blocks of 256 threads up to 131,072 values (50,257: 6.7 us, 7.3 at 512
-// threads, 8.5 at 1024), of 512 past that (3,000,000: 13.3 against 16.0 us).
+// are independent.  V = 1: the plain loop, a value a trip, a memory latency each.  V = 8: eight values requested before
+// any is looked at, the index clamped so that no branch parts the loads (every wave then loads, also past the end).
+// Back to back, V = 1 / V = 8 / many blocks (these 6.1 to 7.5 us from box to box): 100 values 4.1 / 4.1 / 6.8 us, 1,000
+// 4.26 / 4.94 / 6.8, 4,096 4.75 / 5.01 / 7.4, 8,193 5.43 / 5.79 / 7.3, 12,000 6.02 / 6.12 / 7.4, 14,000 6.33 / 6.16 / 7.4, 16,385
+// 6.80 / 6.78 / 7.5, 20,000 7.34 / 7.05 / 6.9, 24,000 8.00 / 7.18 / 7.4, 50,257 12.3 / 11.3 / 7.0, 200,000 - / 34.7 / 8.2, 3,000,000 - / 457 /
+// 13.3.  Many blocks of 256 threads up to 131,072 values (50,257: 6.7 us, 7.3 at 512 threads, 8.5 at 1024), of 512
+// past that (3,000,000: 13.3 against 16.0 us).
 #define RACE_V 8
 __global__ void k_race_none(i64* out) { *out = -1; }
 template <int MANY, int NT, int V = RACE_V>
@@ -1678,17 +1680,26 @@ __global__ __launch_bounds__(NT) void k_stage_race(const i64* v, i64 n, i64* out
     __shared__ i64 bis[NW];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     i64 bv = 0, bi = -1;
-    for (i64 b = (i64)blockIdx.x * (NT * V); b < n; b += (i64)gridDim.x * (NT * V)) {
-        i64 x[V];
-#pragma unroll
-        for (int k = 0; k < V; k++) {
-            const i64 i = b + tid + NT * k;
-            x[k] = v[i < n ? i : n - 1];
+    if constexpr (V == 1) {
+        static_assert(!MANY, "one block");
+        for (i64 i = tid; i < n; i += NT) {
+            const i64 x = v[i];
+            if (bi < 0 || x > bv) { bv = x; bi = i; }
         }
+    } else {
+        const i64 step = MANY ? (i64)gridDim.x * (NT * V) : NT * V;
+        for (i64 b = MANY ? (i64)blockIdx.x * (NT * V) : 0; b < n; b += step) {
+            i64 x[V];
 #pragma unroll
-        for (int k = 0; k < V; k++) {
-            const i64 i = b + tid + NT * k;                 // (grows: a later equal value never wins)
-            if (i < n && (bi < 0 || x[k] > bv)) { bv = x[k]; bi = i; }
+            for (int k = 0; k < V; k++) {
+                const i64 i = b + tid + NT * k;
+                x[k] = v[i < n ? i : n - 1];
+            }
+#pragma unroll
+            for (int k = 0; k < V; k++) {
+                const i64 i = b + tid + NT * k;             // (grows: a later equal value never wins)
+                if (i < n && (bi < 0 || x[k] > bv)) { bv = x[k]; bi = i; }
+            }
         }
     }
 #pragma unroll

@@ -2042,7 +2042,8 @@ extern "C" int sm_tables_destroy(sm_tables* t) {
     return SM_OK;
 }
 
-#define SM_RACE_ONE 16384     // values that one block races (k_stage_race: the two measure equal there)
+#define SM_RACE_PLAIN 12288   // values that one block races a value a trip (k_stage_race's figures)
+#define SM_RACE_ONE 18432     // values that one block races eight a trip (about where the two measure equal)
 static inline int blocks_for(int64_t n, int per) { return (int)((n + per - 1) / per); }
 
 extern "C" int sm_stage_rshift(const int64_t* x, const int64_t* s, int64_t* out, int64_t n, void* stream) {
@@ -2085,7 +2086,7 @@ extern "C" int sm_stage_race(const int64_t* v, int64_t n, int64_t* out_index, vo
     if (n <= 0 || !v || !out_index) return fail(SM_E_ARG, "sm_stage_race: arguments");
     hipStream_t s = (hipStream_t)stream;
     // (an index written over the values themselves is raced by one block, which writes after it has read them)
-    if (n <= 8192) {
+    if (n <= SM_RACE_PLAIN) {
         launch(g_kt.stages, "stage.race", k_stage_race<0, 1024, 1>, dim3(1), dim3(1024), 0, s, (const i64*)v, n, (i64*)out_index);
     } else if (n <= SM_RACE_ONE || (out_index >= v && out_index < v + n)) {
         launch(g_kt.stages, "stage.race", k_stage_race<0, 1024>, dim3(1), dim3(1024), 0, s, (const i64*)v, n, (i64*)out_index);

@@ -1,6 +1,6 @@
-"""sm_stage_race over one block (up to 16,384 values) and many: the largest value, ties to the lowest index
-(base2.py:34-40), at the sizes where the block count and width change, on values that tie across blocks, that are all
-the type's lowest, and with the index written over the values."""
+"""sm_stage_race over one block (up to 18,432 values, from 12,289 on eight a trip) and many: the largest value, ties to
+the lowest index (base2.py:34-40), at the sizes where the block count and width change, on values that tie across
+blocks, that are all the type's lowest, and with the index written over the values."""
 from __future__ import annotations
 
 import numpy as np
@@ -19,7 +19,31 @@ def race(sm, v, out=None, stream=0):
     return int(o[0]) if out is None else int(d[out])
 
 
-@pytest.mark.parametrize("n", [8192, 8193, 16384, 16385, 18431, 18433, 131072, 131073, 1048577, 2100001])
+@pytest.mark.parametrize("n", [1, 63, 64, 1000, 1025])
+def test_few(sm, n):
+    """fewer values than the block has threads, one, and one past a trip"""
+    rng = np.random.default_rng(n)
+    v = rng.integers(-2 ** 62, 2 ** 62, n)
+    assert race(sm, v) == int(v.argmax())
+    assert race(sm, np.full(n, np.iinfo(np.int64).min)) == 0
+    assert race(sm, v, out=n - 1) == int(v.argmax())
+
+
+def test_route(sm):
+    """one launch up to 18,432 values, of the loop that takes a value a trip up to 12,288"""
+    d = torch.zeros(30000, dtype=torch.int64, device="cuda")
+    o = torch.zeros(1, dtype=torch.int64, device="cuda")
+    for n, want in ((1, "k_stage_race<0, 1024, 1>"), (12288, "k_stage_race<0, 1024, 1>"), (12289, "k_stage_race<0, 1024, 8>"),
+                    (18432, "k_stage_race<0, 1024, 8>"), (18433, "k_stage_race<1, 256, 8>")):
+        sm.machine.kernel_times()
+        sm.machine.profile_stages(True)
+        sm.stages.race(d.data_ptr(), n, o.data_ptr())
+        sm.machine.profile_stages(False)
+        got = {k: v[2] for k, v in sm.machine.kernel_times(symbols=True).items() if v[0]}
+        assert want in got["stage.race"] and len(got) == (2 if n > 18432 else 1), (n, got)
+
+
+@pytest.mark.parametrize("n", [12288, 12289, 18432, 8192, 8193, 16384, 16385, 18431, 18433, 131072, 131073, 1048577, 2100001])
 def test_many_blocks(sm, n):
     rng = np.random.default_rng(n)
     v = rng.integers(-2 ** 62, 2 ** 62, n)
