@@ -50,7 +50,7 @@ typedef struct {
                               position but the last runs through the int8 MFMA banks that many rows a pass, each
                               weight read shared by the pass's rows (base2_stream.swift:74-91, 274-275: the
                               prompt through each layer at once); the last position is the first decode step.
-                              64: where more than 64 rows wait, large passes of up to 4096 rows (the machine's
+                              64: where more than 128 rows wait, large passes of up to 4096 rows (the machine's
                               buffers hold min(4096, max_streams x (max_ctx - 1)) rows of 70 KB) */
     int32_t inv;           /* 1: the complement machine (base2_stream.swift:26 `inv`, "the whole machine on the
                               negative"): the stream row, every plate and every light held bit-complemented, each

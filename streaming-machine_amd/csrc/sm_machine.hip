@@ -375,6 +375,7 @@ static const char* BANK[4] = {"qkv", "proj", "fc", "mproj"};
 // The prompt pass in large passes (sm_prompt.hip): its rows' buffers, for cap rows; the streams' own rows (R, QKV,
 // ...) stay the decode steps'.
 #define SM_PROMPT_CAP 4096       // rows a pass at most
+#define SM_PROMPT_FROM 128       // a prompt of more rows takes large passes (run_prefill)
 #define SM_PROMPT_CTX 16384      // (k_pattend's int32 sums hold that many positions)
 struct PromptWS {
     int cap = 0;                                        // 0: no large passes
@@ -1354,7 +1355,10 @@ static int run_prefill(sm_machine* m, int npos) {
     for (int s = 0; s < m->B; s++)
         for (int q = 0; q < npos; q++) m->h_pfmap[(size_t)s * npos + q] = s << 16 | q;
     HIP_TRY(hipMemcpyAsync(m->pfmap, m->h_pfmap.data(), (size_t)total * 4, hipMemcpyHostToDevice, m->st));
-    const bool large = m->pw.cap > 0 && total > chunk;
+    // (two passes of 64 rows are faster than a large one, three are not: a whole call of one stream's 65 / 95 / 128 rows,
+    // GPT-2 1.14 / 1.23 / 1.27 against 1.37 / 1.37 / 1.41 ms, Pythia 1.16 / 1.21 / 1.27 against 1.47 / 1.48 / 1.49; of 129 rows
+    // 1.71 and 1.66 against 1.39 and 1.49; 64 streams' 128 / 192 rows 2.37 / 2.82 against 2.54 / 2.53)
+    const bool large = m->pw.cap > 0 && total > SM_PROMPT_FROM;
     if (large) {
         // whole prompts of as many streams as fit, or a prompt longer than the buffers in parts
         const int per = std::min(m->B, std::max(1, m->pw.cap / npos)), step = std::min(npos, m->pw.cap);
@@ -1625,8 +1629,8 @@ extern "C" int sm_create(const char* layout_dir, const sm_config* cfg, sm_machin
         (rc = dalloc(&m->r_logits, (size_t)m->vocab)) || (rc = dalloc(&m->r_gauge, (size_t)12 * 2 * 768)) ||
         (rc = dalloc(&m->r_fcpre, (size_t)12 * 3072)) || (rc = dalloc(&m->r_hgauge, (size_t)768)))
         return bail(rc);
-    // the large prompt passes' buffers (prefill_rows 64, where a prompt can hold more rows than one small pass)
-    if (mfma && c.prefill_rows == 64 && B * (ctx - 1) > 64 && ctx <= SM_PROMPT_CTX) {
+    // the large prompt passes' buffers (prefill_rows 64, where a prompt can be long enough for them)
+    if (mfma && c.prefill_rows == 64 && B * (ctx - 1) > SM_PROMPT_FROM && ctx <= SM_PROMPT_CTX) {
         PromptWS& w = m->pw;
         const size_t cap = std::min<size_t>(SM_PROMPT_CAP, (B * (ctx - 1) + 127) / 128 * 128);
         const size_t nch = std::max((cap + 63 * B) / PCH + 1, (ctx + PCH - 1) / PCH);

@@ -1,5 +1,5 @@
-"""GPU parity of the large prompt passes (csrc/sm_prompt.hip): with prefill_rows = 64 a prompt of more than 64 rows runs
-in passes of up to 4096 rows, through 128 x 64 MFMA tiles and an attention of 16 query positions a block.  The whole
+"""GPU parity of the large prompt passes (csrc/sm_prompt.hip): with prefill_rows = 64 a prompt of more than 128 rows runs
+in passes of up to 4096 rows, through 64 x 64 MFMA tiles and an attention of 16 query positions a block.  The whole
 cache equals the one that small passes (prefill_rows = 63, pinned to the oracle by test_gpu_prefill.py) leave, at the
 sizes where tiles, chunks of 64 positions and passes end, and the words equal the small passes'."""
 from __future__ import annotations
@@ -45,8 +45,8 @@ def both(sm, d, prompts, n=3):
     return wl
 
 
-# rows of a pass around 64 and the 128-row tile; positions of a slot around the 16-query tile and the 64-position
-# chunk; two passes of whole prompts (20 x 249 rows); one prompt in two parts (4299 rows)
+# rows around one and two passes of 64; positions of a slot around the 64-position chunk; two passes of whole prompts
+# (20 x 249 rows); one prompt in two parts (4299 rows)
 @pytest.mark.parametrize("streams,prompt", [(1, 66), (1, 129), (1, 130), (64, 3), (5, 17), (5, 18), (3, 64), (3, 65), (3, 66),
                                             (2, 300), (20, 250), (1, 4300)])
 def test_gpt2(sm, long_dir, streams, prompt):
@@ -56,6 +56,29 @@ def test_gpt2(sm, long_dir, streams, prompt):
 @pytest.mark.parametrize("streams,prompt", [(1, 66), (4, 18), (3, 66), (2, 300)])
 def test_pythia(sm, py_small_dir, streams, prompt):
     both(sm, py_small_dir, [sm.prompt_ids(200 + s, prompt, 1000) for s in range(streams)])
+
+
+# the line at 128 rows (two passes of 64 up to it), and the edges of queries and chunks past it
+@pytest.mark.parametrize("streams,prompt", [(1, 131), (1, 193), (9, 17), (9, 18), (64, 4), (43, 4)])
+def test_gpt2_past_two_passes(sm, long_dir, streams, prompt):
+    both(sm, long_dir, [sm.prompt_ids(150 + s, prompt, 500) for s in range(streams)])
+
+
+@pytest.mark.parametrize("streams,prompt", [(1, 130), (10, 18), (44, 4)])
+def test_pythia_past_two_passes(sm, py_small_dir, streams, prompt):
+    both(sm, py_small_dir, [sm.prompt_ids(250 + s, prompt, 1000) for s in range(streams)])
+
+
+@pytest.mark.parametrize("kind", ["gpt2", "pythia"])
+def test_route(sm, long_dir, py_small_dir, kind):
+    """a large pass from 129 rows on; 128 rows are two passes of 64"""
+    for streams, prompt, large in ((1, 129, False), (1, 130, True), (64, 3, False), (43, 4, True)):
+        m = sm.Machine(long_dir if kind == "gpt2" else py_small_dir, max_ctx=prompt + 1, max_streams=streams, profile=True)
+        m.kernels()
+        m.streams([sm.prompt_ids(s, prompt, 500) for s in range(streams)], 1)
+        names = m.kernels()
+        m.close()
+        assert any(n.startswith("prompt.") and c for n, (c, _) in names.items()) == large, (streams, prompt, sorted(names))
 
 
 def test_words_of_the_oracle(sm, long_npz, long_dir):
