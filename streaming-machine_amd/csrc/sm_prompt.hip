@@ -442,11 +442,12 @@ __global__ __launch_bounds__(64 * WM * WN * KW, 2) void k_pgemm(PGemmArgs a) {
 //      +32768 held as 32767) is 256 kh + kl' + 128
 //   V  [4 dimension tiles][3 digits][64 lanes][16]: lane l dimension l % 16, byte 4 i + r the position
 //      16 i + 4 (l / 16) + r (the order in which a lane holds its scores); v = d0 + 256 d1 + 65536 d2, each digit
-//      a signed byte
+//      a signed byte (of a value that three do not hold: its three lowest digits)
 //   Q  [4 query tiles][qh, ql][64 lanes][16] and QO [qo]: lane l query l % 16; q = 256 (qh + qo) + ql, digits signed bytes
 //      (qo: the 1 that a digit of 128 passes on)
 // and per position ek, the +32768 mask km, eq, the sum of q; flag[0] bit 0: a value that three digits do not hold,
-// bit 1: a mask is set, bit 2: a qo is; flag[1], flag[2]: the least and the largest ek.
+// bit 1: a mask is set, bit 2: a qo is, bit 3: a value that six digits do not hold; flag[1], flag[2]: the least and
+// the largest ek; Pythia: vmax, the largest |v| of the positions of a wave that holds a value of bit 0 (else 0).
 constexpr int PCH = 64;
 struct PChunk {
     signed char K[4][2][1024];
@@ -454,8 +455,20 @@ struct PChunk {
     signed char Q[4][2][1024];
     i64 km[PCH];
     int ek[PCH], eq[PCH], sq[PCH], flag[PCH];        // flag[0 .. 2]
-    signed char QO[4][1024];                         // written where flag[0] has bit 2
+    signed char QO[4][1024];                         // these two written where flag[0] has bit 0 or bit 2
+    i64 vmax[PCH];
 };
+// the four bytes of four words, by byte: d[k] holds byte k of t[0 .. 3]
+SMD void byte_planes(const unsigned (&t)[4], unsigned (&d)[4]) {
+    const unsigned l01 = __builtin_amdgcn_perm(t[1], t[0], 0x05010400u), l23 = __builtin_amdgcn_perm(t[3], t[2], 0x05010400u);
+    const unsigned h01 = __builtin_amdgcn_perm(t[1], t[0], 0x07030602u), h23 = __builtin_amdgcn_perm(t[3], t[2], 0x07030602u);
+    d[0] = __builtin_amdgcn_perm(l23, l01, 0x05040100u);
+    d[1] = __builtin_amdgcn_perm(l23, l01, 0x07060302u);
+    d[2] = __builtin_amdgcn_perm(h23, h01, 0x05040100u);
+    d[3] = __builtin_amdgcn_perm(h23, h01, 0x07060302u);
+}
+// v without its three lowest signed digits, over 2^24 (modulo 2^40: v modulo 2^64 is those digits and 2^24 times it)
+SMD i64 above3(i64 v) { return (i64)((u64)v + 0x808080u) >> 24; }
 struct PAttArgs {
     AttArgs a;                    // the layer's cache, tables, error word
     PRow x;                       // the qkv rows (strips of PSW)
@@ -491,6 +504,7 @@ __global__ __launch_bounds__(1024) void k_kv_chunk(PAttArgs g) {
         }
     }
     if (threadIdx.x == 0) { ch.flag[0] = 0; ch.flag[1] = INT32_MAX; ch.flag[2] = INT32_MIN; }
+    if (MODEL == 1 && threadIdx.x < PCH) ch.vmax[threadIdx.x] = 0;
     __syncthreads();
     // the OR of a head's two strips (lanes 0-31 hold the one's word, the others the other's), the same in every lane
     auto both = [](i64 o) -> i64 {
@@ -544,7 +558,7 @@ __global__ __launch_bounds__(1024) void k_kv_chunk(PAttArgs g) {
             ekv = a.EK[slotp];
             v[j] = v_whole(a, hrow * a.ctx, p, lane);
         }
-        wide |= (u64)(v[j] + 0x808080) >= 0x1000000ull;
+        wide |= (u64)v[j] + 0x808080u >= 0x1000000u;
         masks |= km != 0;
         emin = min(emin, ekv); emax = max(emax, ekv);
         // q in signed digits; a high digit of 128 as 127 + 1
@@ -559,17 +573,25 @@ __global__ __launch_bounds__(1024) void k_kv_chunk(PAttArgs g) {
         if (lane == 0) { ch.km[pl] = (i64)km; ch.ek[pl] = ekv; ch.eq[pl] = eqv; ch.sq[pl] = sq; }
     }
     // the values' digits: dimension tile lane / 16, lane' = lane % 16 + 16 gq, byte 4 ti + j
-    unsigned t[4];
+    unsigned t[4], dg[4];
 #pragma unroll
-    for (int r = 0; r < 4; r++) t[r] = (unsigned)((int)v[r] + 0x808080);
-    const unsigned l01 = __builtin_amdgcn_perm(t[1], t[0], 0x05010400u), l23 = __builtin_amdgcn_perm(t[3], t[2], 0x05010400u);
-    const unsigned h01 = __builtin_amdgcn_perm(t[1], t[0], 0x07030602u), h23 = __builtin_amdgcn_perm(t[3], t[2], 0x07030602u);
+    for (int r = 0; r < 4; r++) t[r] = (unsigned)v[r] + 0x808080u;
+    byte_planes(t, dg);
     const int o = ((lane & 15) + 16 * gq) * 16 + 4 * ti;
-    *reinterpret_cast<unsigned*>(&ch.V[lane >> 4][0][o]) = __builtin_amdgcn_perm(l23, l01, 0x05040100u) ^ 0x80808080u;
-    *reinterpret_cast<unsigned*>(&ch.V[lane >> 4][1][o]) = __builtin_amdgcn_perm(l23, l01, 0x07060302u) ^ 0x80808080u;
-    *reinterpret_cast<unsigned*>(&ch.V[lane >> 4][2][o]) = __builtin_amdgcn_perm(h23, h01, 0x05040100u) ^ 0x80808080u;
+#pragma unroll
+    for (int k = 0; k < 3; k++) *reinterpret_cast<unsigned*>(&ch.V[lane >> 4][k][o]) = dg[k] ^ 0x80808080u;
     if (!g.ch) return;                                     // (uniform) the last layer: keys and values alone
-    const int fl = (__ballot(wide) ? 1 : 0) | (__ballot(masks) ? 2 : 0) | (__ballot(carry) ? 4 : 0);
+    int fl = (__ballot(wide) ? 1 : 0) | (__ballot(masks) ? 2 : 0) | (__ballot(carry) ? 4 : 0);
+    if (fl & 1) {                                          // (rare) values that three digits do not hold
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            if (__ballot((u64)v[j] + 0x808080808080u >= 0x1000000000000u)) fl |= 8;
+            if (MODEL == 1) {
+                const i64 m = wave_reduce64(iabs64(v[j]), OpMax());
+                if (lane == 0) ch.vmax[4 * wave + j] = m;
+            }
+        }
+    }
     if (lane == 0) {
         if (fl) atomicOr(&ch.flag[0], fl);
         atomicMin(&ch.flag[1], emin);
@@ -579,7 +601,7 @@ __global__ __launch_bounds__(1024) void k_kv_chunk(PAttArgs g) {
     static_assert(sizeof(PChunk) % 16 == 0 && offsetof(PChunk, QO) % 16 == 0, "copied as 16-byte words");
     const v4p* s = reinterpret_cast<const v4p*>(&ch);
     v4p* d = reinterpret_cast<v4p*>(g.ch + ((size_t)slot * 12 + h) * g.nch + c);
-    const int words = (int)((ch.flag[0] & 4 ? sizeof(PChunk) : offsetof(PChunk, QO)) / 16);
+    const int words = (int)((ch.flag[0] & 5 ? sizeof(PChunk) : offsetof(PChunk, QO)) / 16);
     for (int i = threadIdx.x; i < words; i += 1024) d[i] = s[i];
 }
 
@@ -593,9 +615,14 @@ __global__ __launch_bounds__(1024) void k_kv_chunk(PAttArgs g) {
 // arrival, at most 2^24, is three signed digits and a 0/1 fourth, which most chunks lack; the products of equal
 // weight share one int32 accumulator (at most 4 x 2^20 a chunk: callers keep positions below 16384, so none
 // passes 2^31).  The waves' sums meet in LDS in 64 bits.
-// A head with a value that three digits do not hold takes pattend_wide: a query at a time, one wave each.
-// Bound by each wave's chain (keys, products, arrivals' table reads, values) at two waves a SIMD: 36.8 us at one
-// stream's 999 positions, 52.8 at 19 of 212; with the scores in 64 bits throughout 56.5 and 81.
+// A head with a value that three digits do not hold (past 2^23) takes the value sums two or three times: over the three
+// lowest digits of every value, the next three and, with a value past 2^47, the rest, whose digits the waves form from
+// the cache; a sum modulo 2^64 is the groups' sums at 2^0, 2^24 and 2^48.  Two of the four dimension tiles a pass over
+// the chunks there: with four, the kernels spill 20 to 40 vector registers.  A whole call of one 1000-word prompt 2.53 ms
+// with one head of every layer past 2^23, 3.31 with all, 5.76 with all past 2^33, against 2.13 without (15.2, 22.9 and 26.0
+// with a wave walking each query's positions); 19 prompts of 213 words 4.70, 5.92 and 8.79 against 4.43.
+// Bound by each wave's chain (keys, products, arrivals' table reads, values) at two waves a SIMD: 39 us at one
+// stream's 999 positions, 48 at 19 of 212; with the scores in 64 bits throughout 56.5 and 81.
 template <int MODEL>
 SMD i64 patt_score(const AttArgs& a, i64 dot, i64 e) {      // e = eq + ek
     if constexpr (MODEL == 1) return rsh(wmul(dot, a.ehalf), wsub(16, wsub(wmul(e + 10, 65536), a.half) >> 16));
@@ -620,51 +647,11 @@ SMD int pchunk_q(const PChunk* c, int tile, int ql, int d) {
     const int o = (d >> 4) * 256 + ql * 16 + (d & 15);
     return 256 * (c->Q[tile][0][o] + (c->flag[0] & 4 ? c->QO[tile][o] : 0)) + c->Q[tile][1][o];
 }
-template <int MODEL>
-SMD void pattend_wide(const PAttArgs& g, const PChunk* ch, int h, int slot, int p, int lane, int* q_s, int* w_s) {
-    const AttArgs& a = g.a;
-    const PChunk* cq = ch + p / PCH;
-    const size_t hrow = (size_t)(g.s0 + slot) * 12 + h, hb = hrow * a.ctx;
-    q_s[lane] = pchunk_q(cq, (p % PCH) >> 4, p & 15, lane);
-    const i64 eq = cq->eq[p % PCH];
-    auto score = [&](int s) -> i64 {                        // lane's position s <= p against q (LDS, the wave's own)
-        const short* kr = a.K16 + (hb + s) * 64;
-        const u64 km = (u64)a.KM[hb + s];
-        i64 dot = 0;
-        for (int d = 0; d < 64; d++) dot += (i64)q_s[d] * (kr[d] + (int)((km >> d) & 1));
-        return patt_score<MODEL>(a, dot, eq + a.EK[hb + s]);
-    };
-    i64 mx = INT64_MIN;
-    for (int s = lane; s <= p; s += 64) { const i64 v = score(s); mx = v > mx ? v : mx; }
-    mx = wave_reduce64(mx, OpMax());
-    i64 num = 0, z = 0, vm = 0;
-    for (int b = 0; b <= p; b += 64) {
-        const int w = b + lane <= p ? tab_arr(a.tb, wsub(mx, score(b + lane))) : 0;
-        z += w;
-        w_s[lane] = w;
-        for (int s = 0; s < 64 && b + s <= p; s++) {
-            const i64 ws = w_s[s], x = v_whole(a, hb, b + s, lane);
-            num = wadd(num, wmul(ws, x));
-            if (MODEL == 1 && ws) { const i64 ax = iabs64(x); vm = ax > vm ? ax : vm; }
-        }
-    }
-    z = wave_reduce64(z, OpAdd());
-    if (MODEL == 1 && (double)vm * (double)z >= 4611686018427387904.0) atomicOr(a.err, SM_ERR_RANGE);
-    int zt; i64 zm;
-    log2_parts(z, zt, zm);
-    const i64 o = patt_out<MODEL>(a, num, zt, a.tb.LOG2[zm], a.tb.HPOW[zm], true), w = wave_or64(iabs64(o));
-    const size_t r = (size_t)(slot * g.n + p - g.pa);
-    g.out.x32[r * 768 + h * 64 + lane] = (int)o;
-    if (!pnarrow(w)) g.out.x64[r * 768 + h * 64 + lane] = o;
-    if (lane == 0) g.out.orw[r * 12 + h] = w;
-}
-
 template <int MODEL, int NW>
 __global__ __launch_bounds__(64 * NW, 2) void k_pattend(PAttArgs g) {
     const AttArgs& a = g.a;
     __shared__ i64 mx_s[NW][16], z_s[NW][16];
-    __shared__ i64 num_s[NW > 1 ? NW - 1 : 1][NW > 1 ? 16 : 1][64];
-    __shared__ __align__(16) int q_s[NW][64], w_s[NW][64];
+    __shared__ i64 num_s[NW][16][64], vm_s[NW][16];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, ql = lane & 15, pg = lane >> 4;
     const int h = blockIdx.y, slot = blockIdx.z;
     const int p0 = g.pa + 16 * (int)(gridDim.x - 1 - blockIdx.x);     // the longest tiles first
@@ -681,11 +668,6 @@ __global__ __launch_bounds__(64 * NW, 2) void k_pattend(PAttArgs g) {
         emn = min(emn, ch[c].flag[1]); emx = max(emx, ch[c].flag[2]);
     }
     fl = (int)wave_or32((unsigned)fl);
-    if (fl & 1) {                                            // (uniform over the block)
-        for (int i = wave; i < 16 && p0 + i < g.pb; i += NW)
-            pattend_wide<MODEL>(g, ch, h, slot, p0 + i, lane, q_s[wave], w_s[wave]);
-        return;
-    }
     v4p qo = {0, 0, 0, 0};
     if (carry) qo = *reinterpret_cast<const v4p*>(&cq->QO[qt][16 * lane]);
     // the scores in 32 bits (GPT-2): with every shift s = -(eq + ek + 7) in 9..40, rshift(dot, s) is
@@ -696,10 +678,18 @@ __global__ __launch_bounds__(64 * NW, 2) void k_pattend(PAttArgs g) {
     const bool ok32 = MODEL == 0 && !(fl & 2) && __ballot(eql + emx > -16 || eql + emn < -47) == 0;
     // arrivals' sum and digit products (below)
     v4p acc[4][6];
-    i64 z = 0;
+    i64 z = 0, vm = 0;
+    // acc's products of equal weight as 64-bit sums: lane holds dimensions 16 d + 4 pg + r of query ql in [4 d + r]
+    auto sum64 = [&](int d, int r) {
+        u64 n = 0;
+#pragma unroll
+        for (int k = 5; k >= 0; k--) n = (n << 8) + (u64)(i64)acc[d][k][r];
+        return (i64)n;
+    };
     const __amdgpu_buffer_rsrc_t ra = buf_rsrc(a.tb.ARR, (unsigned)a.tb.alen * 4u);   // 0 past the table (base2.py:97)
-    auto body = [&](auto fast) {
-        constexpr bool FAST = decltype(fast)::value;
+    auto body = [&](auto fast, auto wide) {
+        constexpr bool FAST = decltype(fast)::value, WIDE = decltype(wide)::value;
+        constexpr int DN = WIDE ? 2 : 4;                     // dimension tiles a pass over the chunks
         typedef typename std::conditional<FAST, int, i64>::type S;
         constexpr S LOW = FAST ? (S)INT32_MIN : (S)INT64_MIN;
         S sc[16];
@@ -742,12 +732,51 @@ __global__ __launch_bounds__(64 * NW, 2) void k_pattend(PAttArgs g) {
                 }
             }
         };
-        v4p vv[4][3];
-        auto vload = [&](int c) {
+        v4p vv[WIDE ? 1 : 4][3];
+        auto vload = [&](int c, int d) {
 #pragma unroll
-            for (int d = 0; d < 4; d++)
+            for (int k = 0; k < 3; k++) vv[WIDE ? 0 : d][k] = *reinterpret_cast<const v4p*>(&ch[c].V[d][k][16 * lane]);
+        };
+        // WIDE: digits 3 gr .. 3 gr + 2 of chunk c's values, dimension tile d, from the cached rows up to the tile's last
+        // position (past it zeros)
+        auto vform = [&](int c, int d, int gr) {
+            // (the arguments that only this path needs, read here: as the kernel's own they are held in scalar registers
+            // from its start, and the usual path's spill)
+            typedef const __attribute__((address_space(4))) PAttArgs* arg_p;
+            const arg_p ga = (arg_p)__builtin_amdgcn_kernarg_segment_ptr();
+            const size_t hb = ((size_t)(ga->s0 + slot) * 12 + h) * ga->a.ctx;
+            const unsigned n = (unsigned)plast + 1u;
+            const __amdgpu_buffer_rsrc_t rv = buf_rsrc(ga->a.V + hb * 64, n * 256u), rw = buf_rsrc(ga->a.VW + hb, n * 4u),
+                                         r8 = buf_rsrc(ga->a.V64 + hb * 64, n * 512u);
+            int x[16], m[16], any = 0;
 #pragma unroll
-                for (int k = 0; k < 3; k++) vv[d][k] = *reinterpret_cast<const v4p*>(&ch[c].V[d][k][16 * lane]);
+            for (int i = 0; i < 16; i++) {
+                const unsigned s = (unsigned)(PCH * c + 16 * (i >> 2) + 4 * pg + (i & 3));
+                x[i] = buf_load1(rv, (s * 64u + 16u * d + ql) * 4u);
+                m[i] = buf_load1(rw, s * 4u);
+            }
+#pragma unroll
+            for (int i = 0; i < 16; i++) any |= m[i];
+            const bool whole = __ballot(any) != 0;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                unsigned t[4], dg[4];
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    i64 v = x[4 * i + r];
+                    if (whole) {                             // (uniform) rows held whole
+                        const unsigned s = (unsigned)(PCH * c + 16 * i + 4 * pg + r);
+                        const i64 y = buf_load8(r8, m[4 * i + r] ? (s * 64u + 16u * d + ql) * 8u : 0xFFFFFFF0u);
+                        v = m[4 * i + r] ? y : v;
+                    }
+                    v = above3(v);
+                    if (gr == 2) v = above3(v);
+                    t[r] = (unsigned)v + 0x808080u;
+                }
+                byte_planes(t, dg);
+#pragma unroll
+                for (int k = 0; k < 3; k++) vv[0][k][i] = (int)(dg[k] ^ 0x80808080u);
+            }
         };
         // the queries' maxima (base2.py:96): the wave's chunks, the four lane groups, then the waves
         S M = LOW;
@@ -767,120 +796,157 @@ __global__ __launch_bounds__(64 * NW, 2) void k_pattend(PAttArgs g) {
             for (int w = 0; w < NW; w++) { const S x = (S)mx_s[w][ql]; M = x > M ? x : M; }
         }
         // arrivals (base2.py:96-97), their sum, the value sums (base2.py:98): the wave's chunks, last to first
+        const int clast = c, passes = !WIDE ? 1 : (fl & 8 ? 3 : 2) * (4 / DN);
+#pragma unroll 1
+        for (int ps = 0; ps < passes; ps++) {
+            const int gr = WIDE ? ps / (4 / DN) : 0, d0 = WIDE ? ps % (4 / DN) * DN : 0;
+            c = clast;
 #pragma unroll
-        for (int d = 0; d < 4; d++)
+            for (int d = 0; d < DN; d++)
 #pragma unroll
-            for (int k = 0; k < 6; k++) acc[d][k] = v4p{0, 0, 0, 0};
-        while (c >= 0) {
-            if (!FAST) scores(c);                            // (64-bit scores kept over the loop would spill)
-            const int pc = p - PCH * c - 4 * pg;
-            unsigned t[16];
+                for (int k = 0; k < 6; k++) acc[d][k] = v4p{0, 0, 0, 0};
+            while (c >= 0) {
+                if (!FAST) scores(c);                            // (64-bit scores kept over the loop would spill)
+                const int pc = p - PCH * c - 4 * pg;
+                unsigned t[16];
 #pragma unroll
-            for (int i = 0; i < 16; i++) {
-                bool in = 16 * (i >> 2) + (i & 3) <= pc;
-                unsigned d;
-                if constexpr (FAST) {                        // (both below 2^30 in magnitude)
-                    d = (unsigned)(M - sc[i]);
-                    in = in && d < (unsigned)a.tb.alen;
-                } else {
-                    const i64 dd = wsub(M, sc[i]);
-                    in = in && (u64)dd < (u64)a.tb.alen;
-                    d = (unsigned)dd;
+                for (int i = 0; i < 16; i++) {
+                    bool in = 16 * (i >> 2) + (i & 3) <= pc;
+                    unsigned d;
+                    if constexpr (FAST) {                        // (both below 2^30 in magnitude)
+                        d = (unsigned)(M - sc[i]);
+                        in = in && d < (unsigned)a.tb.alen;
+                    } else {
+                        const i64 dd = wsub(M, sc[i]);
+                        in = in && (u64)dd < (u64)a.tb.alen;
+                        d = (unsigned)dd;
+                    }
+                    t[i] = (unsigned)buf_load1(ra, in ? d * 4u : 0xFFFFFFF0u);
                 }
-                t[i] = (unsigned)buf_load1(ra, in ? d * 4u : 0xFFFFFFF0u);
-            }
-            vload(c);
-            unsigned zs = 0;
-            bool top = false;
+                if constexpr (!WIDE) {
 #pragma unroll
-            for (int i = 0; i < 16; i++) {
-                zs += t[i];                                  // at most 16 x 2^24
-                t[i] += 0x808080u;
-                top |= t[i] >> 24 != 0;
-            }
-            z += zs;
-            v4p w0, w1, w2, w3;
+                    for (int d = 0; d < 4; d++) vload(c, d);
+                }
+                unsigned zs = 0;
+                bool top = false;
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const unsigned l01 = __builtin_amdgcn_perm(t[4 * i + 1], t[4 * i], 0x05010400u), l23 = __builtin_amdgcn_perm(t[4 * i + 3], t[4 * i + 2], 0x05010400u);
-                const unsigned h01 = __builtin_amdgcn_perm(t[4 * i + 1], t[4 * i], 0x07030602u), h23 = __builtin_amdgcn_perm(t[4 * i + 3], t[4 * i + 2], 0x07030602u);
-                w0[i] = (int)(__builtin_amdgcn_perm(l23, l01, 0x05040100u) ^ 0x80808080u);
-                w1[i] = (int)(__builtin_amdgcn_perm(l23, l01, 0x07060302u) ^ 0x80808080u);
-                w2[i] = (int)(__builtin_amdgcn_perm(h23, h01, 0x05040100u) ^ 0x80808080u);
-                w3[i] = (int)__builtin_amdgcn_perm(h23, h01, 0x07060302u);
-            }
-            const bool any_top = __ballot(top) != 0;
+                for (int i = 0; i < 16; i++) {
+                    zs += t[i];                                  // at most 16 x 2^24
+                    if (WIDE && MODEL == 1 && (ch[c].flag[0] & 1)) {     // (uniform) the largest |v| that an arrival weighs
+                        const i64 x = ch[c].vmax[16 * (i >> 2) + 4 * pg + (i & 3)];
+                        vm = t[i] && x > vm ? x : vm;
+                    }
+                    t[i] += 0x808080u;
+                    top |= t[i] >> 24 != 0;
+                }
+                if (!WIDE || ps == 0) z += zs;
+                v4p w0, w1, w2, w3;
 #pragma unroll
-            for (int d = 0; d < 4; d++) {
-                acc[d][0] = mfma_i8(vv[d][0], w0, acc[d][0]);
-                acc[d][1] = mfma_i8(vv[d][0], w1, acc[d][1]);
-                acc[d][2] = mfma_i8(vv[d][0], w2, acc[d][2]);
-                acc[d][3] = mfma_i8(vv[d][1], w2, acc[d][3]);
-                acc[d][4] = mfma_i8(vv[d][2], w2, acc[d][4]);
-                acc[d][1] = mfma_i8(vv[d][1], w0, acc[d][1]);
-                acc[d][2] = mfma_i8(vv[d][1], w1, acc[d][2]);
-                acc[d][3] = mfma_i8(vv[d][2], w1, acc[d][3]);
-                acc[d][2] = mfma_i8(vv[d][2], w0, acc[d][2]);
-                if (any_top) {
-                    acc[d][3] = mfma_i8(vv[d][0], w3, acc[d][3]);
-                    acc[d][4] = mfma_i8(vv[d][1], w3, acc[d][4]);
-                    acc[d][5] = mfma_i8(vv[d][2], w3, acc[d][5]);
+                for (int i = 0; i < 4; i++) {
+                    const unsigned ti[4] = {t[4 * i], t[4 * i + 1], t[4 * i + 2], t[4 * i + 3]};
+                    unsigned dg[4];
+                    byte_planes(ti, dg);
+                    w0[i] = (int)(dg[0] ^ 0x80808080u);
+                    w1[i] = (int)(dg[1] ^ 0x80808080u);
+                    w2[i] = (int)(dg[2] ^ 0x80808080u);
+                    w3[i] = (int)dg[3];
+                }
+                const bool any_top = __ballot(top) != 0;
+#pragma unroll
+                for (int d = 0; d < DN; d++) {
+                    if constexpr (WIDE) {
+                        if (gr == 0) vload(c, d0 + d);
+                        else vform(c, d0 + d, gr);
+                    }
+                    const v4p (&x)[3] = vv[WIDE ? 0 : d];
+                    acc[d][0] = mfma_i8(x[0], w0, acc[d][0]);
+                    acc[d][1] = mfma_i8(x[0], w1, acc[d][1]);
+                    acc[d][2] = mfma_i8(x[0], w2, acc[d][2]);
+                    acc[d][3] = mfma_i8(x[1], w2, acc[d][3]);
+                    acc[d][4] = mfma_i8(x[2], w2, acc[d][4]);
+                    acc[d][1] = mfma_i8(x[1], w0, acc[d][1]);
+                    acc[d][2] = mfma_i8(x[1], w1, acc[d][2]);
+                    acc[d][3] = mfma_i8(x[2], w1, acc[d][3]);
+                    acc[d][2] = mfma_i8(x[2], w0, acc[d][2]);
+                    if (any_top) {
+                        acc[d][3] = mfma_i8(x[0], w3, acc[d][3]);
+                        acc[d][4] = mfma_i8(x[1], w3, acc[d][4]);
+                        acc[d][5] = mfma_i8(x[2], w3, acc[d][5]);
+                    }
+                }
+                c -= NW;
+                if (FAST && c >= 0) scores(c);
+            }
+            if constexpr (WIDE) {                                // the groups' sums so far, in the wave's LDS
+#pragma unroll
+                for (int i = 0; i < 4 * DN; i++) {
+                    i64* n = &num_s[wave][4 * d0 + i][lane];
+                    const i64 x = (i64)((u64)sum64(i >> 2, i & 3) << (24 * gr));
+                    *n = gr ? wadd(*n, x) : x;
                 }
             }
-            c -= NW;
-            if (FAST && c >= 0) scores(c);
         }
     };
-    if (ok32) body(Flag<true>{});
-    else body(Flag<false>{});
-    // 64-bit sums: lane holds dimensions 16 d + 4 pg + r of query ql; the waves meet in wave 0
-    i64 num[16];
+    // 64-bit sums; the waves meet in wave 0
+    auto finish = [&](auto wide) {
+        constexpr bool WIDE = decltype(wide)::value;
+        i64 num[16];
 #pragma unroll
-    for (int d = 0; d < 4; d++)
+        for (int i = 0; i < 16; i++) num[i] = WIDE ? num_s[wave][i][lane] : sum64(i >> 2, i & 3);
+        z += __shfl_xor(z, 16, 64);
+        z += __shfl_xor(z, 32, 64);
+        if (WIDE && MODEL == 1)
 #pragma unroll
-        for (int r = 0; r < 4; r++) {
-            u64 n = 0;
+            for (int o = 16; o < 64; o <<= 1) { const i64 x = __shfl_xor(vm, o, 64); vm = x > vm ? x : vm; }
+        if constexpr (NW > 1) {
+            if (wave > 0) {
+                if (lane < 16) z_s[wave][lane] = z;
+                if (WIDE && MODEL == 1 && lane < 16) vm_s[wave][lane] = vm;
+                if (!WIDE)
 #pragma unroll
-            for (int k = 5; k >= 0; k--) n = (n << 8) + (u64)(i64)acc[d][k][r];
-            num[4 * d + r] = (i64)n;
+                    for (int i = 0; i < 16; i++) num_s[wave][i][lane] = num[i];
+            }
+            __syncthreads();
+            if (wave > 0) return;
+#pragma unroll
+            for (int w = 1; w < NW; w++) {
+                z += z_s[w][ql];
+                if (WIDE && MODEL == 1) { const i64 x = vm_s[w][ql]; vm = x > vm ? x : vm; }
+#pragma unroll
+                for (int i = 0; i < 16; i++) num[i] = wadd(num[i], num_s[w][i][lane]);
+            }
         }
-    z += __shfl_xor(z, 16, 64);
-    z += __shfl_xor(z, 32, 64);
-    if constexpr (NW > 1) {
-        if (wave > 0) {
-            if (lane < 16) z_s[wave][lane] = z;
+        const bool live = p < g.pb;
+        // (pythia_base2.py:139; values that three digits hold stay below 2^61 whatever the arrivals)
+        if (WIDE && MODEL == 1 && live && (double)vm * (double)z >= 4611686018427387904.0) atomicOr(a.err, SM_ERR_RANGE);
+        int zt; i64 zm;
+        log2_parts(z, zt, zm);
+        const i64 lg = a.tb.LOG2[zm], hp = a.tb.HPOW[zm];
+        i64 w = 0;
 #pragma unroll
-            for (int i = 0; i < 16; i++) num_s[wave - 1][i][lane] = num[i];
+        for (int i = 0; i < 16; i++) {
+            num[i] = patt_out<MODEL>(a, num[i], zt, lg, hp, live);
+            w |= iabs64(num[i]);
         }
-        __syncthreads();
-        if (wave > 0) return;
+        w |= __shfl_xor(w, 16, 64);
+        w |= __shfl_xor(w, 32, 64);
+        if (!live) return;
+        const size_t r = (size_t)(slot * g.n + p - g.pa), at = r * 768 + h * 64 + 4 * pg;
+        if (pg == 0) g.out.orw[r * 12 + h] = w;
 #pragma unroll
-        for (int w = 1; w < NW; w++) {
-            z += z_s[w][ql];
+        for (int d = 0; d < 4; d++) {
+            *reinterpret_cast<v4p*>(g.out.x32 + at + 16 * d) = v4p{(int)num[4 * d], (int)num[4 * d + 1], (int)num[4 * d + 2], (int)num[4 * d + 3]};
+            if (!pnarrow(w))
 #pragma unroll
-            for (int i = 0; i < 16; i++) num[i] = wadd(num[i], num_s[w - 1][i][lane]);
+                for (int r4 = 0; r4 < 4; r4++) g.out.x64[at + 16 * d + r4] = num[4 * d + r4];
         }
+    };
+    if (__builtin_expect(fl & 1, 0)) {                        // (uniform over the block)
+        body(Flag<false>{}, Flag<true>{});
+        finish(Flag<true>{});
+        return;
     }
-    int zt; i64 zm;
-    log2_parts(z, zt, zm);
-    const i64 lg = a.tb.LOG2[zm], hp = a.tb.HPOW[zm];
-    const bool live = p < g.pb;
-    i64 w = 0;
-#pragma unroll
-    for (int i = 0; i < 16; i++) {
-        num[i] = patt_out<MODEL>(a, num[i], zt, lg, hp, live);
-        w |= iabs64(num[i]);
-    }
-    w |= __shfl_xor(w, 16, 64);
-    w |= __shfl_xor(w, 32, 64);
-    if (!live) return;
-    const size_t r = (size_t)(slot * g.n + p - g.pa), at = r * 768 + h * 64 + 4 * pg;
-    if (pg == 0) g.out.orw[r * 12 + h] = w;
-#pragma unroll
-    for (int d = 0; d < 4; d++) {
-        *reinterpret_cast<v4p*>(g.out.x32 + at + 16 * d) = v4p{(int)num[4 * d], (int)num[4 * d + 1], (int)num[4 * d + 2], (int)num[4 * d + 3]};
-        if (!pnarrow(w))
-#pragma unroll
-            for (int r4 = 0; r4 < 4; r4++) g.out.x64[at + 16 * d + r4] = num[4 * d + r4];
-    }
+    if (ok32) body(Flag<true>{}, Flag<false>{});
+    else body(Flag<false>{}, Flag<false>{});
+    finish(Flag<false>{});
 }

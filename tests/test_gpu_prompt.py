@@ -125,6 +125,70 @@ def test_planted(sm, long_npz, tmp_path_factory, plant):
         m.close()
 
 
+@pytest.mark.parametrize("shift", [7, 15, 31, 45])
+def test_wide_values(sm, long_npz, tmp_path_factory, shift):
+    """a head whose value columns are scaled by 2^shift, of both signs and every size up to about 2^(18 + shift): some
+    rows three digits hold and some they do not (7), 32 bits do (15), 32 bits do not, some past 2^47 (31), all of 64 bits
+    (45, where the sums wrap as int64 sums do); a second head past 2^23 throughout"""
+    import oracle
+    npz = dict(long_npz)
+    e, b = npz["qkv.0.e"].copy(), npz["qkv.0.b"].copy()
+    e[1536 + 5 * 64:1536 + 6 * 64] += shift
+    b[1536 + 9 * 64:1536 + 10 * 64] -= 1 << 23
+    npz["qkv.0.e"], npz["qkv.0.b"] = e, b
+    d = sm.layout(npz, str(tmp_path_factory.mktemp("wide")))
+    prompts = [sm.prompt_ids(450 + s, 140, 500) for s in range(2)]
+    words = both(sm, d, prompts)
+    orc = oracle.Oracle(npz, bound=False)
+    for s, p in enumerate(prompts):
+        assert words[s].tolist() == orc.generate(p, 3, 160)
+
+
+@pytest.mark.parametrize("plant", ["value 24 bits", "value 50 bits", "key"])
+def test_planted_earlier_pass(sm, long_npz, tmp_path_factory, plant):
+    """a prompt of two parts (4199 rows): the second part's queries against the first part's values past 24 and 50 bits
+    and its keys of +32768, which come back from the cache"""
+    npz = dict(long_npz)
+    b = npz["qkv.0.b"].copy()
+    if plant == "key":
+        b[768 + 64 + 3] = (1 << 40) - (1 << 23)
+    else:
+        b[1536:1600] += ((1 << 23) if plant == "value 24 bits" else (1 << 50)) + np.arange(64, dtype=np.int64) * (1 << 18)
+    npz["qkv.0.b"] = b
+    both(sm, sm.layout(npz, str(tmp_path_factory.mktemp("earlier"))), [sm.prompt_ids(470, 4200, 500)])
+
+
+def test_pythia_earlier_pass(sm, tmp_path_factory):
+    """the Pythia machine's prompt of two parts, one head's values past 24 bits"""
+    sd, cfg = sm.pythia.random_pythia(seed=5, vocab=1000)
+    npz = sm.pythia.convert_pythia(sd, dict(cfg, n_ctx=4300))
+    e = np.array(npz["qkv.0.e"]).copy()
+    e[128:192] += 8
+    npz["qkv.0.e"] = e
+    both(sm, sm.pythia.pythia_layout(npz, str(tmp_path_factory.mktemp("py_earlier"))), [sm.prompt_ids(480, 4200, 1000)])
+
+
+def test_wide_head_time(sm, long_npz, long_dir, tmp_path_factory):
+    """one head past 2^23 in every layer leaves the attention of a long prompt within ten times what it takes without
+    (its value sums run twice, their digits formed from the cache; a walk over the positions, a query a wave, took 30)"""
+    npz = dict(long_npz)
+    for l in range(12):
+        b = npz[f"qkv.{l}.b"].copy()
+        b[1536:1600] += 1 << 23
+        npz[f"qkv.{l}.b"] = b
+    wide = sm.layout(npz, str(tmp_path_factory.mktemp("wide_time")))
+    us = []
+    for d in (long_dir, wide):
+        m = sm.Machine(d, max_ctx=1001, profile=True)
+        for _ in range(3):
+            m.kernels()
+            m.stream(sm.prompt_ids(490, 1000, 500), 1)
+            n, t = m.kernels()["prompt.attend"]
+        us.append(n * t)
+        m.close()
+    assert us[1] < 10 * us[0], us
+
+
 @pytest.mark.parametrize("shift", [12, 16])
 def test_pythia_wide_values(sm, py_small_npz, tmp_path_factory, shift):
     """the Pythia machine with a head whose value columns are scaled by 2^shift.  Its values then lie below about
