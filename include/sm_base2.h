@@ -50,8 +50,10 @@ typedef struct {
                               position but the last runs through the int8 MFMA banks that many rows a pass, each
                               weight read shared by the pass's rows (base2_stream.swift:74-91, 274-275: the
                               prompt through each layer at once); the last position is the first decode step.
-                              64: where more than 128 rows wait, large passes of up to 4096 rows (the machine's
-                              buffers hold min(4096, max_streams x (max_ctx - 1)) rows of 70 KB) */
+                              64: where more than 128 rows wait, large passes of up to 4096 rows.  Their buffers
+                              are allocated at create, for min(4096, max_streams x (max_ctx - 1)) rows where that
+                              passes 128: about 100 KB a row and 0.4 MB a stream.  Where they do not fit, and with
+                              prefill_rows 63, there are none and every prompt takes small passes */
     int32_t inv;           /* 1: the complement machine (base2_stream.swift:26 `inv`, "the whole machine on the
                               negative"): the stream row, every plate and every light held bit-complemented, each
                               pile corrected by the plate's column sum, the light's sum and the input count, stream

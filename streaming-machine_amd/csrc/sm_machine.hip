@@ -559,6 +559,30 @@ static int parse_norms(const std::string& text, std::vector<std::pair<std::strin
     return SM_OK;
 }
 
+static void prompt_free(PromptWS& w) {
+    void* pp[] = {w.R, w.qkv.x32, w.qkv.x64, w.qkv.orw, w.att.x32, w.att.x64, w.att.orw, w.hid.x32, w.hid.x64, w.hid.orw,
+                  w.pl[0], w.pl[1], w.pl[2], w.ri[0], w.ri[1], w.ri[2], w.ch};
+    for (void* p : pp) hfree(p);
+    w = PromptWS();
+}
+// The large prompt passes' buffers, asked for after everything else a machine holds: where they do not fit, prompts take
+// passes of 64 rows, which need none of them.
+static void prompt_alloc(sm_machine* m) {
+    PromptWS& w = m->pw;
+    const size_t B = m->B, ctx = m->ctx;
+    const size_t cap = std::min<size_t>(SM_PROMPT_CAP, (B * (ctx - 1) + 127) / 128 * 128);
+    const size_t nch = std::max((cap + 63 * B) / PCH + 1, (ctx + PCH - 1) / PCH);
+    auto prow = [&](PRow& r, size_t n, size_t sw) { return dalloc(&r.x32, cap * n) || dalloc(&r.x64, cap * n) || dalloc(&r.orw, cap * n / sw); };
+    if (dalloc(&w.R, cap * 768) || prow(w.qkv, 2304, PSW) || prow(w.att, 768, 64) || prow(w.hid, 3072, PSW) ||
+        dalloc(&w.pl[0], cap * 768 * 3) || (m->kind == 1 && dalloc(&w.pl[1], cap * 768 * 3)) || dalloc(&w.pl[2], cap * 3072 * 3) ||
+        dalloc(&w.ri[0], cap * 8) || dalloc(&w.ri[1], cap * 8) || dalloc(&w.ri[2], cap * 8) || dalloc(&w.ch, nch * 12)) {
+        prompt_free(w);
+        (void)hipGetLastError();               // (not the next call's error)
+        return;
+    }
+    w.cap = (int)cap;
+}
+
 static void machine_free(sm_machine* m) {
     if (!m) return;
     for (int i = 0; i < 6; i++)
@@ -578,9 +602,7 @@ static void machine_free(sm_machine* m) {
                   m->top_hi, m->top_lo, m->cand_j, m->cand_h, m->cand_c, m->top_x, m->top_f, m->top_n, m->top_w,
                   m->top_pile, m->top_score, m->asc, m->acm, m->aacc, m->V64, m->VW, m->vbig};
     for (void* p : ps) hfree(p);
-    PromptWS& w = m->pw;
-    void* pp[] = {w.R, w.qkv.x32, w.qkv.x64, w.qkv.orw, w.att.x32, w.att.x64, w.att.orw, w.hid.x32, w.hid.x64, w.hid.orw, w.pl[0], w.pl[1], w.pl[2], w.ri[0], w.ri[1], w.ri[2], w.ch};
-    for (void* p : pp) hfree(p);
+    prompt_free(m->pw);
     for (int l = 0; l < 12; l++)
         for (int j = 0; j < 2; j++) { hfree(m->ng[l][j]); hfree(m->nb[l][j]); }
     if (m->hpin) (void)hipHostFree(m->hpin);
@@ -1629,24 +1651,6 @@ extern "C" int sm_create(const char* layout_dir, const sm_config* cfg, sm_machin
         (rc = dalloc(&m->r_logits, (size_t)m->vocab)) || (rc = dalloc(&m->r_gauge, (size_t)12 * 2 * 768)) ||
         (rc = dalloc(&m->r_fcpre, (size_t)12 * 3072)) || (rc = dalloc(&m->r_hgauge, (size_t)768)))
         return bail(rc);
-    // the large prompt passes' buffers (prefill_rows 64, where a prompt can be long enough for them)
-    if (mfma && c.prefill_rows == 64 && B * (ctx - 1) > SM_PROMPT_FROM && ctx <= SM_PROMPT_CTX) {
-        PromptWS& w = m->pw;
-        const size_t cap = std::min<size_t>(SM_PROMPT_CAP, (B * (ctx - 1) + 127) / 128 * 128);
-        const size_t nch = std::max((cap + 63 * B) / PCH + 1, (ctx + PCH - 1) / PCH);
-        auto prow = [&](PRow& r, size_t n, size_t sw) -> int {
-            int e;
-            if ((e = dalloc(&r.x32, cap * n)) || (e = dalloc(&r.x64, cap * n)) || (e = dalloc(&r.orw, cap * n / sw))) return e;
-            return SM_OK;
-        };
-        if ((rc = dalloc(&w.R, cap * 768)) || (rc = prow(w.qkv, 2304, PSW)) || (rc = prow(w.att, 768, 64)) ||
-            (rc = prow(w.hid, 3072, PSW)) || (rc = dalloc(&w.pl[0], cap * 768 * 3)) ||
-            (py && (rc = dalloc(&w.pl[1], cap * 768 * 3))) || (rc = dalloc(&w.pl[2], cap * 3072 * 3)) ||
-            (rc = dalloc(&w.ri[0], cap * 8)) || (rc = dalloc(&w.ri[1], cap * 8)) || (rc = dalloc(&w.ri[2], cap * 8)) ||
-            (rc = dalloc(&w.ch, nch * 12)))
-            return bail(rc);
-        w.cap = (int)cap;
-    }
     // rows with a value past 32 bits whole beside their low 32 bits (the float arrival keeps the int32 cache and its
     // error)
     if (!m->farr && ((rc = dalloc(&m->V64, 12 * B * ctx * 768)) || (rc = dalloc(&m->VW, 12 * B * ctx * 12)) ||
@@ -1664,6 +1668,8 @@ extern "C" int sm_create(const char* layout_dir, const sm_config* cfg, sm_machin
         m->hpin = nullptr;
         return bail(fail(SM_E_OOM, "hipHostMalloc: the generate readback buffer"));
     }
+    // (where a prompt can be long enough for them, run_prefill)
+    if (mfma && c.prefill_rows == 64 && B * (ctx - 1) > SM_PROMPT_FROM && ctx <= SM_PROMPT_CTX) prompt_alloc(m);
     m->prompts.assign(B, {});
     m->gsteps = c.graph_steps > 0 ? c.graph_steps : 16;
     if ((rc = sm_reset(m))) return bail(rc);
