@@ -284,7 +284,8 @@ struct sm_tables {
     i64 log768 = 0, eps40 = 0;
     int verified = 0;         // every entry equals its defining formula (checked on the device at create)
     int* scratch = nullptr;   // [4..7] mismatch counts
-    int* posn = nullptr;      // [SM_STAGE_ATT_CTX] the numbers 0, 1, ..: the attention entry points' positions
+    // the attention entry points' (stage_init)
+    int* posn = nullptr;      // [SM_STAGE_ATT_CTX] the numbers 0, 1, ..: their positions
     int* herr = nullptr;      // pinned host memory, SM_ERR_SLOTS lines: a call's error word (StageErr)
     mutable std::atomic<unsigned> next{0};                    // where a call looks for a free line
     mutable std::atomic<bool> taken[SM_ERR_SLOTS] = {};       // the lines that calls in flight hold
@@ -331,16 +332,6 @@ static int tables_init(sm_tables& T, const i64* phi, const i64* arr, int alen, c
     }
     if ((rc = dalloc(&T.scratch, 16))) return rc;
     HIP_TRY(hipMemset(T.scratch, 0, 64));
-    {
-        std::vector<int> n(SM_STAGE_ATT_CTX);
-        for (int i = 0; i < SM_STAGE_ATT_CTX; i++) n[i] = i;
-        if ((rc = dalloc(&T.posn, n.size()))) return rc;
-        HIP_TRY(hipMemcpy(T.posn, n.data(), n.size() * 4, hipMemcpyHostToDevice));
-        if (hipHostMalloc(&T.herr, SM_ERR_SLOTS * 64, hipHostMallocDefault) != hipSuccess) {
-            T.herr = nullptr;
-            return fail(SM_E_OOM, "hipHostMalloc: the error word");
-        }
-    }
     T.alen = alen; T.log768 = log768; T.eps40 = eps40;
     // every entry against its formula (table_mode 1 refuses tables that are not the reference's)
     const int n = alen + 1 > 65536 ? alen + 1 : 65536;
@@ -349,6 +340,20 @@ static int tables_init(sm_tables& T, const i64* phi, const i64* arr, int alen, c
     unsigned bad[4];
     HIP_TRY(hipMemcpy(bad, T.scratch + 4, sizeof(bad), hipMemcpyDeviceToHost));
     T.verified = (bad[0] | bad[1] | bad[2] | bad[3]) == 0;
+    return SM_OK;
+}
+
+// what the attention entry points keep with their tables (a machine's own have no use for it)
+static int stage_init(sm_tables& T) {
+    std::vector<int> n(SM_STAGE_ATT_CTX);
+    for (int i = 0; i < SM_STAGE_ATT_CTX; i++) n[i] = i;
+    int rc;
+    if ((rc = dalloc(&T.posn, n.size()))) return rc;
+    HIP_TRY(hipMemcpy(T.posn, n.data(), n.size() * 4, hipMemcpyHostToDevice));
+    if (hipHostMalloc(&T.herr, SM_ERR_SLOTS * 64, hipHostMallocDefault) != hipSuccess) {
+        T.herr = nullptr;
+        return fail(SM_E_OOM, "hipHostMalloc: the error words");
+    }
     return SM_OK;
 }
 
@@ -2037,6 +2042,7 @@ extern "C" int sm_tables_create(const int64_t* phi, const int64_t* arrival, int3
     if (!phi || !arrival || !log2t || !exp2t || !out) return fail(SM_E_ARG, "sm_tables_create: null argument");
     sm_tables* t = new sm_tables();
     int rc = tables_init(*t, (const i64*)phi, (const i64*)arrival, alen, (const i64*)log2t, (const i64*)exp2t, log2_768, eps40);
+    if (!rc) rc = stage_init(*t);
     if (rc) { tables_free(*t); delete t; return rc; }
     *out = t;
     return SM_OK;
