@@ -814,7 +814,7 @@ __global__ __launch_bounds__(64 * NW, 2) void k_pattend(PAttArgs g) {
                     bool in = 16 * (i >> 2) + (i & 3) <= pc;
                     unsigned d;
                     if constexpr (FAST) {                        // (both below 2^30 in magnitude)
-                        d = (unsigned)(M - sc[i]);
+                        d = (unsigned)M - (unsigned)sc[i];   // (past p LOW: wraps, and is not in)
                         in = in && d < (unsigned)a.tb.alen;
                     } else {
                         const i64 dd = wsub(M, sc[i]);
