@@ -489,6 +489,7 @@ __global__ __launch_bounds__(1024) void k_kv_chunk(PAttArgs g) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, ti = wave >> 2, gq = wave & 3;   // 16-position tile, group
     const size_t hrow = (size_t)st * 12 + h;
     const bool fresh = PCH * c >= g.pa;
+    if (!fresh && !g.ch) return;                           // (the last layer: an earlier pass's chunk has nothing to do)
     auto at = [&](int part) { return MODEL == 1 ? h * 192 + part * 64 + lane : part * 768 + h * 64 + lane; };
     i64 q[4], k[4], v[4], oq[4], ok[4], ov[4];
 #pragma unroll
