@@ -980,7 +980,9 @@ SMD void v_store(const AttArgs& a, size_t hrow, int p, int lane, i64 x) {
             if (wide) atomicOr(a.vbig + hrow, 1);
         }
     } else if (wide && lane == 0) {
-        *a.err = SM_ERR_V32;                                // (the stage entry points: a word of host memory)
+        // (a plain store: only the stage entry points come here, whose word is host memory and takes this one bit; every
+        // machine that stores values through v_store has V64, and the float arrival's own kernel keeps its error word)
+        *a.err = SM_ERR_V32;
     }
 }
 // The (stream, head)'s mark of values past 32 bits (vbig), as a vector load issued with the cached rows and waited
