@@ -1068,9 +1068,11 @@ static int launch_step_pythia_batched(sm_machine* m, int parts, int nrows = 0,
             // the attention), four launches a layer with proj and the row kernel
             launch(m->cfg.profile, "fc+qkv", k_gemm_pair<EPI_PLAIN_EDGE, EPI_PLAIN>, dim3(gf * RT + gq * RT), dim3(256), 0,
                    m->st, af, aq, gf * RT, gf, gq);
-            // mproj's column tiles a block: three, or RT at one and two row tiles, 192 blocks, while those and the
-            // attention's fit two blocks a CU (2 streams 276 against 285 us a step, 24 streams 322 against 333; at 32
-            // streams, 576 blocks, 362 against 338)
+            // mproj's column tiles a block: three, or two while the launch's blocks then fit the GPU as they do with
+            // three: at one row tile one block a CU (96 of mproj's; a step at context 48 / 300 with one, two, three
+            // tiles: 2 streams 263 / 314, 264 / 313, 268 / 314 us, 8 streams 295 / 333, 284 / 326, 288 / 325; 14 streams,
+            // 264 blocks, 299 / 341, 303 / 347, 295 / 337), at two row tiles two a CU (192 of mproj's; 24 streams, two
+            // and three tiles, 310 / 383 and 320 / 387; 32 streams, 576 blocks, 362 and 338)
             auto pair = [&](auto nb) {
                 constexpr int NB = decltype(nb)::value;
                 const int gm = m->mbank[l][3].ntiles / NB * 4;
@@ -1081,7 +1083,7 @@ static int launch_step_pythia_batched(sm_machine* m, int parts, int nrows = 0,
                     launch(m->cfg.profile, "attend+mproj.part", k_attend_mproj<1, 0, NB>, dim3(12 * B + gm * RT), dim3(256),
                            (size_t)m->ctx * 12, m->st, at, am, 12 * B, gm);
             };
-            if (RT < 3 && 12 * B + 192 <= 512) pair(std::integral_constant<int, RT < 3 ? RT : 3>{});
+            if (RT < 3 && 12 * B + 96 * RT <= 256 * RT) pair(std::integral_constant<int, RT < 3 ? 2 : 3>{});
             else pair(std::integral_constant<int, 3>{});
         } else {
             launch(m->cfg.profile, "qkv", k_gemm<768, 1, 1, EPI_PLAIN>, dim3(gq, RT), dim3(256), 0, m->st, aq);

@@ -156,6 +156,21 @@ def test_small_model_batched_record(sm, py_small_dir, py_small_oracle, pgolden, 
     m.close()
 
 
+@pytest.mark.parametrize("B,tiles", [(2, 2), (13, 2), (14, 3), (16, 3), (17, 2), (26, 2), (27, 3)])
+def test_paired_mproj_tiles(sm, py_small_dir, py_small_oracle, B, tiles):
+    """the column tiles a block of the launch that mproj shares with the attention, at the stream counts where they change,
+    and the words there"""
+    prompts = [sm.prompt_ids(160 + s, 6, 1000) for s in range(B)]
+    m = sm.Machine(py_small_dir, max_ctx=32, max_streams=B, profile=True)
+    sm.machine.kernel_times()
+    words = m.streams(prompts, 4)
+    sym = sm.machine.kernel_times(symbols=True)["attend+mproj.part"][2]
+    m.close()
+    assert f", {tiles}>" in sym, sym
+    for s in (0, B - 1):
+        assert words[s] == py_small_oracle.generate(prompts[s], 4, 32)
+
+
 def test_pythia_32_streams_64_token_prompts(sm, py_full_dir, py_full_npz, pgolden):
     """32 streams of 64-word prompts: the two golden streams, a sample against the oracle, a late stream's cache"""
     from oracle.pythia import PythiaOracle
