@@ -2303,11 +2303,14 @@ static void rows_product(const sm_plate* p, const int64_t* x16, int32_t rows, in
         // columns of every row; below, where that leaves CUs idle, the head's kernel.  Back to back, this bank / that
         // kernel: 16 rows 11.1 / 12.6 us at 16,000 columns, 25.6 / 27.5 at 50,257; 32 rows 13.2 / 13.6 and 30.6 / 35.9;
         // 64 rows 18.1 / 16.1 and 38.5 / 39.8, 31.1 / 35.9 at 40,001 (8,000 columns: 17.2 / 12.8)
-        if (P.N >= (RT <= 2 ? 16000 : 36000)) {
+        // One row of 49,153 to 51,456 columns stays with the head's kernel: the bank's last blocks past three a CU take a
+        // round of their own there (17.1 / 17.9 us at 50,257 columns; two rows 17.9 / 17.9)
+        const int blocks = (P.ntiles + 3) / 4;
+        if (P.N >= (RT <= 2 ? 16000 : 36000) && !(rows == 1 && blocks > 768 && blocks <= 804)) {
             PGemmArgs pa{};
             pa.N = P.N; pa.rows = rows; pa.W = P.W; pa.csum = P.csum; pa.we = P.e; pa.bias = P.b;
             pa.planes = planes; pa.rowinfo = rowinfo; pa.Y = (i64*)pile;
-            const dim3 grid((unsigned)((P.ntiles + 3) / 4 + 7) / 8 * 8);
+            const dim3 grid((unsigned)(blocks + 7) / 8 * 8);
             launch(timed, "plate.head_rows", k_pgemm<768, EPI_PILE, RT <= 2 ? 2 : 4, 4, 2, 2, 2>, grid, dim3(256), 0, s, pa);
         } else if (P.N > 3072) {
             launch(timed, "plate.head_rows", k_head_rows<RT, EPI_PILE>, dim3(head_rows_grid(P.ntiles)), dim3(256), 0, s, ga);

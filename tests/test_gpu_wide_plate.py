@@ -30,3 +30,22 @@ def test_piles(sm, nout):
             # float64 products: every partial sum below 2^40
             assert torch.equal(pile, (dx.double() @ wd).to(torch.int64)), (rows, call.__name__)
     plate.close()
+
+
+@pytest.mark.parametrize("nout,rows,bank", [(49152, 1, True), (49153, 1, False), (51456, 1, False), (51457, 1, True), (49153, 2, True),
+                                            (15999, 1, False), (16000, 1, True), (36000, 33, True), (35999, 33, False)])
+def test_route(sm, nout, rows, bank):
+    """which kernel a row count and width take, and its piles"""
+    rng = np.random.default_rng(nout + rows)
+    w = rng.integers(-32768, 32768, (768, nout)).astype(np.int16)
+    plate = sm.Plate(w, np.zeros(nout, np.int32), np.zeros(nout, np.int64), tile_cols=0)
+    dx = torch.from_numpy(rng.integers(-32768, 32769, (rows, 768))).cuda()
+    pile = torch.full((rows, nout), -1, dtype=torch.int64, device="cuda")
+    sm.machine.kernel_times()
+    sm.machine.profile_stages(True)
+    plate.product_rows(dx.data_ptr(), rows, pile.data_ptr())
+    sm.machine.profile_stages(False)
+    sym = sm.machine.kernel_times(symbols=True)["plate.head_rows"][2]
+    assert ("k_pgemm" in sym) == bank, sym
+    assert torch.equal(pile, (dx.double() @ torch.from_numpy(w).cuda().double()).to(torch.int64))
+    plate.close()
