@@ -2,14 +2,14 @@
 // (base2_stream.swift:74-91, 274-275 sends the whole prompt through each layer).  A pass holds `rows` rows, row
 // r = slot n + (position - a) for S streams (slots) of n = b - a positions [a, b) each: whole prompts of several
 // streams (a = 0), or part of one longer prompt (a a multiple of PCH).  Every number is the decode step's.
-//   k_pgemm     a bank over all rows (base2.py:29-32): 128 x 64 output tiles of int8 MFMA over byte planes
+//   k_pgemm     a bank over all rows (base2.py:29-32): 64 x 64 output tiles of int8 MFMA over byte planes
 //   k_kv_chunk  the pass's q, k, v of one head (base2.py:93) into the cache, and, for the pass's attention, the
 //               byte planes of 64 positions in MFMA operand order
 //   k_pattend   attention (base2.py:94-99) of 16 query positions a block, scores and value sums by MFMA
 //   k_plight    the rows' lights (base2.py:24-27, 55-60); the Pythia machine's two gauges are k_py_rows'
 // Why: in passes of 64 rows each launch (5-9 us, latency-bound) serves 64 rows, and the attention, one block a (head,
-// row), reads a row's whole cache for one query.  Same box, a whole call: GPT-2, one 1000-word prompt 9.40 -> 2.14 ms;
-// 19 prompts of 213 words and 17 words each 39.2 -> 12.4 ms; 64 prompts of 32 words and 128 words 85.8 -> 73.0 ms.
+// row), reads a row's whole cache for one query.  Same box, a whole call: GPT-2, one 1000-word prompt 9.40 -> 2.13 ms;
+// 19 prompts of 213 words and 17 words each 39.2 -> 12.3 ms; 64 prompts of 32 words and 128 words 85.8 -> 72.7 ms.
 #include "sm_kernels.h"
 #include <cstddef>
 #include <type_traits>
@@ -176,6 +176,8 @@ __global__ __launch_bounds__(512) void k_plight(PLightArgs a) {
 // in MFMA order, so every global load and LDS access is a whole wave's consecutive 1 KB.  Blocks are numbered so that
 // each XCD (block index % 8) works on a contiguous run of row tiles.  KW = 2: two groups of such waves, each every
 // second k step, whose sums meet in LDS (half the chain of a 3072-wide bank with few blocks).
+// Bound by neither unit: at 999 / 4,028 rows fc keeps the matrix units 16 / 23 % busy, mproj 18 / 32 %, and the LDS units as
+// much, with no bank conflicts; its waves wait 30 to 40 % of their cycles, mostly on memory and barriers.
 // The machine's tiles are 64 x 64 (four waves of 32 x 32, 126 registers, four blocks a CU): at 999 / 4,028 rows fc
 // takes 23.4 / 73 us and mproj 26.5 / 59 us with one group (0.7-1.3 POP/s of int8).  128 x 64 tiles measured 28.8 / 79 and 35.9 / 69
 // us, 128 x 128 of eight waves 26.8 / 77 and 44.6 / 69, 128 x 128 of four waves 39 / 111 and 67 / 100 (fewer blocks to
