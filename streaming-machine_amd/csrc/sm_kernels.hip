@@ -1665,16 +1665,15 @@ __global__ __launch_bounds__(NTHR) void k_stage_rows(const i64* X, int n, int ga
 }
 // The race over n values: largest, ties to the lowest index (base2.py:34-40).
 // MANY = 0: one block, which writes its winner.  MANY = 1: blocks in a grid stride, each then putting its winner into
-// *out where it beats the one that is there (*out is -1 on entry, k_race_none): no scratch, so calls on any streams
-// are independent.  V = 1: the plain loop, a value a trip, a memory latency each.  V = 8: eight values requested before
+// *out where it beats the one that is there: no scratch, so calls on any streams are independent.  What *out holds on
+// entry needs no clearing (a launch of its own, 2 us of a lone call): no index of v, it loses to any; an index of v, it
+// is one of the values raced and loses to the winner like the others.  V = 1: the plain loop, a value a trip, a memory latency each.  V = 8: eight values requested before
 // any is looked at, the index clamped so that no branch parts the loads (every wave then loads, also past the end).
-// Back to back, V = 1 / V = 8 / many blocks (these 6.1 to 7.5 us from box to box): 100 values 4.1 / 4.1 / 6.8 us, 1,000
-// 4.26 / 4.94 / 6.8, 4,096 4.75 / 5.01 / 7.4, 8,193 5.43 / 5.79 / 7.3, 12,000 6.02 / 6.12 / 7.4, 14,000 6.33 / 6.16 / 7.4, 16,385
-// 6.80 / 6.78 / 7.5, 20,000 7.34 / 7.05 / 6.9, 24,000 8.00 / 7.18 / 7.4, 50,257 12.3 / 11.3 / 7.0, 200,000 - / 34.7 / 8.2, 3,000,000 - / 457 /
-// 13.3.  Many blocks of 256 threads up to 131,072 values (50,257: 6.7 us, 7.3 at 512 threads, 8.5 at 1024), of 512
-// past that (3,000,000: 13.3 against 16.0 us).
+// Back to back on rows in turn, V = 1 / V = 8 / many blocks: 500 values 4.1 / 4.2 / 4.3 us, 1,000 4.24 / 4.93 / 4.23, 2,000 4.42 /
+// 4.94 / 4.23, 4,000 4.73 / 5.02 / 4.22, 8,193 5.40 / 5.81 / 4.53, 16,385 6.7 / 6.7 / 4.95, 24,000 8.1 / 7.3 / 5.1, 50,257 12.4 /
+// 11.3 / 5.5 (7.0 with the launch that cleared *out), 131,072 45 / 24 / 6.1, 1,000,000 318 / 154 / 11.1.  Many blocks of 256 threads
+// up to 131,072 values, of 512 past that (3,000,000: 13.3 against 16.0 us).
 #define RACE_V 8
-__global__ void k_race_none(i64* out) { *out = -1; }
 template <int MANY, int NT, int V = RACE_V>
 __global__ __launch_bounds__(NT) void k_stage_race(const i64* v, i64 n, i64* out) {
     constexpr int NW = NT / 64;
@@ -1718,9 +1717,9 @@ __global__ __launch_bounds__(NT) void k_stage_race(const i64* v, i64 n, i64* out
         if constexpr (MANY) {
             u64* o = reinterpret_cast<u64*>(out);
             u64 cur = atomicAdd(o, 0ull);
-            // (each failed exchange means that another block's winner came in: at most gridDim.x of them.  An index
-            // that is no index of v, the -1 or one from a race of other values that a caller lets share the word, is
-            // replaced and never read through)
+            // (each failed exchange means that another block's winner came in: at most gridDim.x of them.  What is no
+            // index of v, from before or from a race of other values that a caller lets share the word, is replaced and
+            // never read through)
             while (cur >= (u64)n || bv > v[cur] || (bv == v[cur] && (u64)bi < cur)) {
                 const u64 old = atomicCAS(o, cur, (u64)bi);
                 if (old == cur) break;

@@ -2078,8 +2078,8 @@ extern "C" int sm_tables_destroy(sm_tables* t) {
     return SM_OK;
 }
 
-#define SM_RACE_PLAIN 12288   // values that one block races a value a trip (k_stage_race's figures)
-#define SM_RACE_ONE 18432     // values that one block races eight a trip (about where the two measure equal)
+#define SM_RACE_PLAIN 1024    // values that one block races in one trip (k_stage_race's figures: many blocks are faster past it)
+#define SM_RACE_INPLACE 12288 // the same where the index is written over the values: past it eight a trip
 static inline int blocks_for(int64_t n, int per) { return (int)((n + per - 1) / per); }
 
 extern "C" int sm_stage_rshift(const int64_t* x, const int64_t* s, int64_t* out, int64_t n, void* stream) {
@@ -2122,12 +2122,12 @@ extern "C" int sm_stage_race(const int64_t* v, int64_t n, int64_t* out_index, vo
     if (n <= 0 || !v || !out_index) return fail(SM_E_ARG, "sm_stage_race: arguments");
     hipStream_t s = (hipStream_t)stream;
     // (an index written over the values themselves is raced by one block, which writes after it has read them)
-    if (n <= SM_RACE_PLAIN) {
+    const bool inplace = out_index >= v && out_index < v + n;
+    if (n <= (inplace ? SM_RACE_INPLACE : SM_RACE_PLAIN)) {
         launch(g_kt.stages, "stage.race", k_stage_race<0, 1024, 1>, dim3(1), dim3(1024), 0, s, (const i64*)v, n, (i64*)out_index);
-    } else if (n <= SM_RACE_ONE || (out_index >= v && out_index < v + n)) {
+    } else if (inplace) {
         launch(g_kt.stages, "stage.race", k_stage_race<0, 1024>, dim3(1), dim3(1024), 0, s, (const i64*)v, n, (i64*)out_index);
     } else {
-        launch(g_kt.stages, "stage.race.none", k_race_none, dim3(1), dim3(1), 0, s, (i64*)out_index);
         const int nt = n <= 131072 ? 256 : 512;
         const unsigned blocks = (unsigned)std::min<int64_t>(256, (n + nt * RACE_V - 1) / (nt * RACE_V));
         if (nt == 256) launch(g_kt.stages, "stage.race", k_stage_race<1, 256>, dim3(blocks), dim3(256), 0, s, (const i64*)v, n, (i64*)out_index);

@@ -1,6 +1,6 @@
-"""sm_stage_race over one block (up to 18,432 values, from 12,289 on eight a trip) and many: the largest value, ties to
-the lowest index (base2.py:34-40), at the sizes where the block count and width change, on values that tie across
-blocks, that are all the type's lowest, and with the index written over the values."""
+"""sm_stage_race over one block (up to 1,024 values, and with the index written over the values) and many: the largest
+value, ties to the lowest index (base2.py:34-40), at the sizes where the block count and width change, on values that tie
+across blocks, that are all the type's lowest, and with the index written over the values."""
 from __future__ import annotations
 
 import numpy as np
@@ -19,9 +19,9 @@ def race(sm, v, out=None, stream=0):
     return int(o[0]) if out is None else int(d[out])
 
 
-@pytest.mark.parametrize("n", [1, 63, 64, 1000, 1025])
+@pytest.mark.parametrize("n", [1, 63, 64, 1000, 1023, 1024, 1025, 1026, 2047, 2048, 2049, 4097])
 def test_few(sm, n):
-    """fewer values than the block has threads, one, and one past a trip"""
+    """fewer values than a block has threads, one, and values on both sides of a trip and of a block's share"""
     rng = np.random.default_rng(n)
     v = rng.integers(-2 ** 62, 2 ** 62, n)
     assert race(sm, v) == int(v.argmax())
@@ -30,17 +30,19 @@ def test_few(sm, n):
 
 
 def test_route(sm):
-    """one launch up to 18,432 values, of the loop that takes a value a trip up to 12,288"""
-    d = torch.zeros(30000, dtype=torch.int64, device="cuda")
+    """one launch each: of one block up to 1,024 values and, where the index is written over them, at any count, a value a
+    trip up to 12,288; else of many"""
+    d = torch.zeros(140000, dtype=torch.int64, device="cuda")
     o = torch.zeros(1, dtype=torch.int64, device="cuda")
-    for n, want in ((1, "k_stage_race<0, 1024, 1>"), (12288, "k_stage_race<0, 1024, 1>"), (12289, "k_stage_race<0, 1024, 8>"),
-                    (18432, "k_stage_race<0, 1024, 8>"), (18433, "k_stage_race<1, 256, 8>")):
+    one, eight = "k_stage_race<0, 1024, 1>", "k_stage_race<0, 1024, 8>"
+    for n, out, want in ((1, o, one), (1024, o, one), (1025, o, "k_stage_race<1, 256, 8>"), (131072, o, "k_stage_race<1, 256, 8>"),
+                         (131073, o, "k_stage_race<1, 512, 8>"), (12288, d, one), (12289, d, eight), (131073, d, eight)):
         sm.machine.kernel_times()
         sm.machine.profile_stages(True)
-        sm.stages.race(d.data_ptr(), n, o.data_ptr())
+        sm.stages.race(d.data_ptr(), n, out.data_ptr())
         sm.machine.profile_stages(False)
-        got = {k: v[2] for k, v in sm.machine.kernel_times(symbols=True).items() if v[0]}
-        assert want in got["stage.race"] and len(got) == (2 if n > 18432 else 1), (n, got)
+        got = {k: v for k, v in sm.machine.kernel_times(symbols=True).items() if v[0]}
+        assert list(got) == ["stage.race"] and got["stage.race"][0] == 1 and want in got["stage.race"][2], (n, got)
 
 
 @pytest.mark.parametrize("n", [12288, 12289, 18432, 8192, 8193, 16384, 16385, 18431, 18433, 131072, 131073, 1048577, 2100001])
@@ -57,6 +59,21 @@ def test_many_blocks(sm, n):
     low[n - 1] += 1
     assert race(sm, low) == n - 1
     assert race(sm, v, out=n // 2) == 0                        # the index over a value: written after it is read
+
+
+@pytest.mark.parametrize("n", [1025, 2049, 18433, 50257, 1048577])
+def test_word_before(sm, n):
+    """the output word before the call: a losing index, the winner, a tied higher index, the value count, -1, the type's ends"""
+    rng = np.random.default_rng(n + 1)
+    v = rng.integers(-2 ** 40, 2 ** 40, n)
+    v[[n // 3, n // 2, n - 1]] = 2 ** 41
+    d = torch.from_numpy(v).cuda()
+    for before in (0, int(v.argmin()), n // 3, n // 2, n - 1, n, -1, 2 ** 62, -2 ** 63):
+        o = torch.full((1,), before, dtype=torch.int64, device="cuda")
+        for _ in range(3):
+            sm.stages.race(d.data_ptr(), n, o.data_ptr())
+            torch.cuda.synchronize()
+            assert int(o[0]) == n // 3, before
 
 
 def test_two_streams(sm):
